@@ -217,8 +217,9 @@ int wkv7_backward_ex(const void *weight_decay, const void *receptance,
  * waits. A wait that gives up
  * (which a correct kernel never does) makes the launch overwrite every output
  * of that (batch, head) -- output, removal_state, the checkpoints, the final
- * state -- with NaN, and adds one to a counter on the device. No counterpart
- * in the reference. wkv7_take_faults waits for `stream`, stores in *count the
+ * state -- with NaN, and adds one to a counter on the device. So does a call
+ * cut into segments, whichever of its passes gave up (a backward's first pass
+ * has such waits too: its gradients then). No counterpart in the reference. wkv7_take_faults waits for `stream`, stores in *count the
  * number of such events on the current device since the previous call,
  * resets the counter, and returns WKV7_ERR_HANDOVER if *count > 0 (WKV7_OK
  * otherwise). Calls on one device must not overlap. */

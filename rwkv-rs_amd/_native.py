@@ -1,5 +1,4 @@
-"""ctypes binding of libwkv7_hip.so, the C ABI declared in include/wkv7.h and
-include/rwkv_neighbors.h.
+"""ctypes binding of libwkv7_hip.so, the C ABI declared in include/.
 
 The library is built in-tree by rwkv-rs_amd/build.py. Loading fails loudly when
 it is missing: there is no fallback implementation.
@@ -54,6 +53,10 @@ EXPORTS = (
     "rwkv_cross_entropy_l2wrap_forward", "rwkv_cross_entropy_l2wrap_backward",
 )
 
+# and those of include/wkv7_segments.h
+SEGMENT_EXPORTS = ("wkv7_forward_workspace_bytes", "wkv7_backward_workspace_bytes",
+                   "wkv7_forward_ws", "wkv7_backward_ws")
+
 _P = ctypes.c_void_p
 _I64 = ctypes.c_int64
 _INT = ctypes.c_int
@@ -67,6 +70,10 @@ _SIGNATURES = {
     "wkv7_backward": ([_P] * 10 + [_I64] * 5 + [_INT] * 3 + [_P] * 8, _INT),
     "wkv7_forward_ex": ([_P] * 7 + [_I64] * 5 + [_INT] * 3 + [_P] * 6, _INT),
     "wkv7_backward_ex": ([_P] * 10 + [_I64] * 5 + [_INT] * 3 + [_P] * 9, _INT),
+    "wkv7_forward_workspace_bytes": ([_I64] * 5 + [_INT, _P], _I64),
+    "wkv7_backward_workspace_bytes": ([_I64] * 5 + [_INT, _P], _I64),
+    "wkv7_forward_ws": ([_P] * 7 + [_I64] * 5 + [_INT] * 3 + [_P] * 6 + [_I64, _P], _INT),
+    "wkv7_backward_ws": ([_P] * 10 + [_I64] * 5 + [_INT] * 3 + [_P] * 9 + [_I64, _P], _INT),
     "wkv7_take_faults": ([_P, _P], _INT),
     "wkv7_pretrain_forward": ([_P] * 6 + [_I64] * 5 + [_INT] + [_P] * 4, _INT),
     "wkv7_pretrain_backward": ([_P] * 9 + [_I64] * 5 + [_INT] + [_P] * 7, _INT),

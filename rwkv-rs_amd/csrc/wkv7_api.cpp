@@ -5,6 +5,7 @@
 // indexing does not match its buffers. The reference panics on the same
 // conditions (wkv7_common/host.rs:109-112 and the unwraps at :175, :358).
 #include "../../include/wkv7.h"
+#include "../../include/wkv7_segments.h"
 
 #include <hip/hip_runtime.h>
 
@@ -90,6 +91,47 @@ int kernel_choice(const wkv7_options* o, wkv7::KernelChoice* kc) {
   kc->step_only = o->kernels == WKV7_KERNELS_STEP;
   kc->spin_limit = o->handover_spin_limit;
   return WKV7_OK;
+}
+
+// a launch descriptor's shape, without its buffers
+template <typename Desc>
+Desc call_shape(const Shape& sh, int dtype, const wkv7::KernelChoice& kc) {
+  Desc d{};
+  d.dtype = static_cast<wkv7::Dtype>(dtype);
+  d.B = static_cast<int>(sh.B);
+  d.T = static_cast<int>(sh.T);
+  d.H = static_cast<int>(sh.H);
+  d.C = static_cast<int>(sh.C);
+  d.kc = kc;
+  return d;
+}
+
+template <typename Desc>
+int64_t workspace_bytes(int64_t B, int64_t T, int64_t H, int64_t N, int64_t C, int dtype,
+                        const wkv7_options* options) {
+  wkv7::KernelChoice kc;
+  if (kernel_choice(options, &kc) || check_shape(B, T, H, N, C, dtype)) return -1;
+  const auto d = call_shape<Desc>(Shape{B, T, H, C}, dtype, kc);
+  return wkv7::segment_bytes(wkv7::plan_segments(d), d.B, d.H);
+}
+
+// the workspace is written, so it counts among the outputs
+int check_workspace(void* workspace, int64_t bytes, std::vector<Range>* outs) {
+  if (!workspace) return WKV7_OK;
+  if (bytes < 0) return WKV7_ERR_SHAPE;
+  if (!aligned(workspace, 16)) return WKV7_ERR_ALIGNMENT;
+  outs->push_back({workspace, bytes});
+  return WKV7_OK;
+}
+
+// cut the call into segments if the workspace holds what that takes
+template <typename Desc>
+void take_workspace(Desc* d, void* workspace, int64_t bytes) {
+  if (!workspace) return;
+  const wkv7::Segments s = wkv7::plan_segments(*d);
+  if (s.G < 2 || bytes < wkv7::segment_bytes(s, d->B, d->H)) return;
+  d->seg = s;
+  wkv7::place_segments(&d->seg, d->B, d->H, workspace);
 }
 
 }  // namespace
@@ -179,6 +221,33 @@ int wkv7_forward_ex(const void* weight_decay, const void* receptance, const void
                     int use_initial_state, int return_final_state, float* state,
                     float* removal_state, void* output, float* final_state,
                     const wkv7_options* options, void* stream) {
+  return wkv7_forward_ws(weight_decay, receptance, key, value, removal, replacement,
+                         initial_state, batch_size, context_len, num_heads, head_size,
+                         chunk_len, dtype, use_initial_state, return_final_state, state,
+                         removal_state, output, final_state, options, nullptr, 0, stream);
+}
+
+int64_t wkv7_forward_workspace_bytes(int64_t batch_size, int64_t context_len,
+                                     int64_t num_heads, int64_t head_size, int64_t chunk_len,
+                                     int dtype, const wkv7_options* options) {
+  return workspace_bytes<wkv7::ForwardDesc>(batch_size, context_len, num_heads, head_size,
+                                            chunk_len, dtype, options);
+}
+int64_t wkv7_backward_workspace_bytes(int64_t batch_size, int64_t context_len,
+                                      int64_t num_heads, int64_t head_size, int64_t chunk_len,
+                                      int dtype, const wkv7_options* options) {
+  return workspace_bytes<wkv7::BackwardDesc>(batch_size, context_len, num_heads, head_size,
+                                             chunk_len, dtype, options);
+}
+
+int wkv7_forward_ws(const void* weight_decay, const void* receptance, const void* key,
+                    const void* value, const void* removal, const void* replacement,
+                    const float* initial_state, int64_t batch_size, int64_t context_len,
+                    int64_t num_heads, int64_t head_size, int64_t chunk_len, int dtype,
+                    int use_initial_state, int return_final_state, float* state,
+                    float* removal_state, void* output, float* final_state,
+                    const wkv7_options* options, void* workspace, int64_t workspace_bytes,
+                    void* stream) {
   wkv7::KernelChoice kc;
   if (int rc = kernel_choice(options, &kc)) return rc;
   if (int rc = check_shape(batch_size, context_len, num_heads, head_size, chunk_len, dtype))
@@ -212,22 +281,18 @@ int wkv7_forward_ex(const void* weight_decay, const void* receptance, const void
                              {removal_state, sh.tok_elems() * 4},
                              {output, tok}};
   if (return_final_state) outs.push_back({final_state, st});
+  if (int rc = check_workspace(workspace, workspace_bytes, &outs)) return rc;
   if (any_overlap(outs, ins)) return WKV7_ERR_OVERLAP;
   if (sh.state_elems() == 0) return WKV7_OK;
 
-  wkv7::ForwardDesc d;
-  d.dtype = static_cast<wkv7::Dtype>(dtype);
-  d.B = static_cast<int>(batch_size);
-  d.T = static_cast<int>(context_len);
-  d.H = static_cast<int>(num_heads);
-  d.C = static_cast<int>(chunk_len);
+  auto d = call_shape<wkv7::ForwardDesc>(sh, dtype, kc);
   d.w = weight_decay; d.r = receptance; d.k = key; d.v = value; d.a = removal; d.b = replacement;
   d.s0 = use_initial_state ? initial_state : nullptr;
   d.ckpt = state;
   d.sa = removal_state;
   d.y = output;
   d.sT = return_final_state ? final_state : nullptr;
-  d.kc = kc;
+  take_workspace(&d, workspace, workspace_bytes);
   return hip_status(wkv7::launch_forward(d, static_cast<hipStream_t>(stream)));
 }
 
@@ -257,6 +322,24 @@ int wkv7_backward_ex(const void* weight_decay, const void* receptance, const voi
                      void* weight_decay_grad, void* receptance_grad, void* key_grad,
                      void* value_grad, void* removal_grad, void* replacement_grad,
                      float* initial_state_grad, const wkv7_options* options, void* stream) {
+  return wkv7_backward_ws(weight_decay, receptance, key, value, removal, replacement, state,
+                          removal_state, output_grad, final_state_grad, batch_size, context_len,
+                          num_heads, head_size, chunk_len, dtype, use_final_state_grad,
+                          write_initial_state_grad, weight_decay_grad, receptance_grad,
+                          key_grad, value_grad, removal_grad, replacement_grad,
+                          initial_state_grad, options, nullptr, 0, stream);
+}
+
+int wkv7_backward_ws(const void* weight_decay, const void* receptance, const void* key,
+                     const void* value, const void* removal, const void* replacement,
+                     const float* state, const float* removal_state, const void* output_grad,
+                     const float* final_state_grad, int64_t batch_size, int64_t context_len,
+                     int64_t num_heads, int64_t head_size, int64_t chunk_len, int dtype,
+                     int use_final_state_grad, int write_initial_state_grad,
+                     void* weight_decay_grad, void* receptance_grad, void* key_grad,
+                     void* value_grad, void* removal_grad, void* replacement_grad,
+                     float* initial_state_grad, const wkv7_options* options, void* workspace,
+                     int64_t workspace_bytes, void* stream) {
   wkv7::KernelChoice kc;
   if (int rc = kernel_choice(options, &kc)) return rc;
   if (int rc = check_shape(batch_size, context_len, num_heads, head_size, chunk_len, dtype))
@@ -296,15 +379,11 @@ int wkv7_backward_ex(const void* weight_decay, const void* receptance, const voi
   std::vector<Range> outs;
   for (void* p : grads) outs.push_back({p, tok});
   if (write_initial_state_grad) outs.push_back({initial_state_grad, st});
+  if (int rc = check_workspace(workspace, workspace_bytes, &outs)) return rc;
   if (any_overlap(outs, ins)) return WKV7_ERR_OVERLAP;
   if (sh.state_elems() == 0) return WKV7_OK;
 
-  wkv7::BackwardDesc d;
-  d.dtype = static_cast<wkv7::Dtype>(dtype);
-  d.B = static_cast<int>(batch_size);
-  d.T = static_cast<int>(context_len);
-  d.H = static_cast<int>(num_heads);
-  d.C = static_cast<int>(chunk_len);
+  auto d = call_shape<wkv7::BackwardDesc>(sh, dtype, kc);
   d.w = weight_decay; d.r = receptance; d.k = key; d.v = value; d.a = removal; d.b = replacement;
   d.ckpt = state;
   d.sa = removal_state;
@@ -313,7 +392,7 @@ int wkv7_backward_ex(const void* weight_decay, const void* receptance, const voi
   d.dw = weight_decay_grad; d.dr = receptance_grad; d.dk = key_grad; d.dv = value_grad;
   d.da = removal_grad; d.db = replacement_grad;
   d.ds0 = write_initial_state_grad ? initial_state_grad : nullptr;
-  d.kc = kc;
+  take_workspace(&d, workspace, workspace_bytes);
   return hip_status(wkv7::launch_backward(d, static_cast<hipStream_t>(stream)));
 }
 

@@ -301,5 +301,22 @@ __device__ __forceinline__ void lds_acquire() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// every output of one (batch, head) of a forward to NaN, by the threads of a
+// workgroup
+template <typename Tio>
+__device__ __forceinline__ void poison_forward(Tio* y, float* sa, float* ckpt, float* sT, int64_t b, int64_t h,
+                                               int64_t H, int64_t T, int64_t nck, int tid, int threads) {
+  const float nan = __builtin_nanf("");
+  const int64_t bh = b * H + h;
+  for (int64_t i = tid; i < T * kHead; i += threads) {
+    const int64_t off = ((b * T + (i >> 6)) * H + h) * kHead + (i & 63);
+    Io<Tio>::put1(&y[off], nan);
+    sa[off] = nan;
+  }
+  for (int64_t i = tid; i < nck * kHead * kHead; i += threads) ckpt[bh * nck * (kHead * kHead) + i] = nan;
+  if (sT)
+    for (int i = tid; i < kHead * kHead; i += threads) sT[bh * (kHead * kHead) + i] = nan;
+}
+
 }  // namespace chunk
 }  // namespace wkv7

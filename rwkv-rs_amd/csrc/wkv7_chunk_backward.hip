@@ -125,6 +125,11 @@ struct BwdChunkParams {
   float* ds0;                  // [B,H,64,64] or null
   int T, H;
   int C;                       // chunk_len: a multiple of 16
+  // segmented calls only:
+  int cps;                     // chunks per segment
+  const float* bound;          // segment g < G - 1 of [B,H,G,64,64]: the state gradient at its end
+  const int* fault;            // [B,H,G]: a boundary gradient is not there
+  unsigned int* faults;        // the device's counter of such events
 };
 
 // element (row, key) of a staged gradient tile: 16-byte pieces rotated by
@@ -256,7 +261,14 @@ __device__ __forceinline__ void setup_products(Prep& P, const GramIn& g, int wav
 // kLong: chunk_len > 16. Only every (chunk_len / 16)-th start state is a
 // checkpoint; the others are rebuilt by the reference's reversal (see
 // reverse_chunk), on the set-up waves.
-template <bool kLong>
+//
+// kSeg: grid (H, B, G), workgroup (h, b, g) runs segment g of the sequence,
+// chunks g cps .. With chunk_len > 16 a segment is a whole number of
+// checkpoint intervals. A sequence in one piece has an instance of its own:
+// through the segmented one it took 1% longer (841 against 828 us at B=8,
+// T=4096, H=32; the segment's bounds and fault words cost four spilled
+// registers).
+template <bool kLong, bool kSeg>
 __global__ __launch_bounds__(kBlock, 1) void wkv7_bwd_chunk_kernel(const BwdChunkParams p) {
   __shared__ BwdLds L;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -269,7 +281,25 @@ __global__ __launch_bounds__(kBlock, 1) void wkv7_bwd_chunk_kernel(const BwdChun
   const int64_t bh = (int64_t)b * H + h;
   const int64_t tstride = (int64_t)H * kHead;
   const int64_t tok0 = ((int64_t)b * T * H + h) * kHead;
-  const int nchunks = T / kL;
+  const int g = kSeg ? blockIdx.z : 0, G = kSeg ? gridDim.z : 1;
+  // this segment's chunks, in reverse
+  const int first = g * p.cps, last = kSeg ? min(first + p.cps, T / kL) - 1 : T / kL - 1;
+  if (kSeg) {
+    // a boundary gradient that a given-up hand-over wait left unformed: every
+    // gradient of the (batch, head) is NaN, and the event is counted
+    bool bad = false;
+    for (int i = 1; i < G; ++i) bad |= p.fault[bh * G + i] != 0;
+    if (bad) {
+      for (int i = tid; i < (last + 1 - first) * kL * kHead; i += kBlock) {
+        const int64_t off = tok0 + (int64_t)(kL * first + (i >> 6)) * tstride + (i & 63);
+        p.dw[off] = p.dr[off] = p.dk[off] = p.dv[off] = p.da[off] = p.db[off] = 0x7fc0;
+      }
+      if (first == 0 && tid == 0) atomicAdd(p.faults, 1u);
+      if (p.ds0 && first == 0)
+        for (int i = tid; i < kHead * kHead; i += kBlock) p.ds0[bh * (kHead * kHead) + i] = __builtin_nanf("");
+      return;
+    }
+  }
   const int q = kLong ? p.C / kL : 1;   // 16-step chunks per checkpoint
   const float* const ckbh = p.ckpt + bh * (T / (kL * q)) * (kHead * kHead);
 
@@ -326,11 +356,13 @@ __global__ __launch_bounds__(kBlock, 1) void wkv7_bwd_chunk_kernel(const BwdChun
   // ---- state gradient (gradient waves): value tile jb = wq, key tiles ib,
   // result layout (rows = key i = 16 ib + 4 qd + r, columns = value j = 16 jb + t)
   const int jb = wq, jcol = 16 * jb + t;
+  const float* const dsE = kSeg && g < G - 1 ? p.bound + (bh * G + g) * (kHead * kHead)
+                         : p.dsT ? p.dsT + bh * (kHead * kHead) : nullptr;
   f32x4 dS[4];
 #pragma unroll
   for (int ib = 0; ib < 4; ++ib) {
-    if (grad && p.dsT)
-      dS[ib] = *reinterpret_cast<const f32x4*>(p.dsT + bh * (kHead * kHead) + jcol * kHead + 16 * ib + 4 * qd);
+    if (grad && dsE)
+      dS[ib] = *reinterpret_cast<const f32x4*>(dsE + jcol * kHead + 16 * ib + 4 * qd);
     else
       dS[ib] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
@@ -381,9 +413,9 @@ __global__ __launch_bounds__(kBlock, 1) void wkv7_bwd_chunk_kernel(const BwdChun
     }
   };
   // kLong, set-up waves: the start state of the chunk processed last, i.e.
-  // the end state of the next one (the last checkpoint before the loop)
+  // the end state of the next one (the segment's last checkpoint before the loop)
   f32x4 Snext[2][2];
-  if (kLong && !grad) load_ckpt(T / (kL * q) - 1, Snext);
+  if (kLong && !grad) load_ckpt((last + 1) / q - 1, Snext);
 
   // the staged gradient tiles of chunk cc to memory (gradient waves in the
   // loop, whose phase B is the shorter one; set-up waves after it): thread
@@ -427,7 +459,6 @@ __global__ __launch_bounds__(kBlock, 1) void wkv7_bwd_chunk_kernel(const BwdChun
   if (!grad) __builtin_amdgcn_s_setprio(2);
 
   // ---- prologue: set up the last chunk (set-up waves)
-  const int last = nchunks - 1;
   if (!grad) {
     reinterpret_cast<uint2*>(&L.zero[0][0])[utid] = make_uint2(0, 0);
     const Pre pr = fetch(last, last);
@@ -798,14 +829,16 @@ __global__ __launch_bounds__(kBlock, 1) void wkv7_bwd_chunk_kernel(const BwdChun
       }
     }
   };
-  for (int c = last; c >= 1; --c) run_chunk(c, std::true_type{});
-  run_chunk(0, std::false_type{});
+  // a segment that does not start the sequence sets up the chunk before its
+  // first one along with it, for nothing, which keeps one loop body
+  for (int c = last; c >= first && c >= 1; --c) run_chunk(c, std::true_type{});
+  if (first == 0) run_chunk(0, std::false_type{});
 
   lds_barrier();
-  if (!grad) finish(0);
+  if (!grad) finish(first);
   lds_barrier();
-  if (!grad) flush(0);
-  if (grad && p.ds0) {
+  if (!grad) flush(first);
+  if (grad && p.ds0 && first == 0) {
 #pragma unroll
     for (int ib = 0; ib < 4; ++ib)
       *reinterpret_cast<f32x4*>(p.ds0 + bh * (kHead * kHead) + jcol * kHead + 16 * ib + 4 * qd) = dS[ib];
@@ -840,11 +873,19 @@ hipError_t launch_backward_chunked(const BackwardDesc& d, hipStream_t stream) {
   p.T = d.T;
   p.H = d.H;
   p.C = d.C;
-  const dim3 grid(d.H, d.B, 1), block(kBlock, 1, 1);
-  if (d.C == kL)
-    hipLaunchKernelGGL(wkv7_bwd_chunk_kernel<false>, grid, block, 0, stream, p);
-  else
-    hipLaunchKernelGGL(wkv7_bwd_chunk_kernel<true>, grid, block, 0, stream, p);
+  p.cps = d.seg.cps;
+  p.bound = d.seg.bound;
+  p.fault = d.seg.fault;
+  p.faults = nullptr;
+  const dim3 grid(d.H, d.B, d.seg.G), block(kBlock, 1, 1);
+  if (d.seg.G > 1) {
+    if (hipError_t e = handover_fault_counter(&p.faults)) return e;
+    if (hipError_t e = launch_segment_bounds(d, stream)) return e;
+  }
+  auto* const kernel = d.seg.G > 1
+      ? (d.C == kL ? wkv7_bwd_chunk_kernel<false, true> : wkv7_bwd_chunk_kernel<true, true>)
+      : (d.C == kL ? wkv7_bwd_chunk_kernel<false, false> : wkv7_bwd_chunk_kernel<true, false>);
+  hipLaunchKernelGGL(kernel, grid, block, 0, stream, p);
   return hipGetLastError();
 }
 

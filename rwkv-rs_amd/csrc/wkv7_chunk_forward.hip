@@ -74,7 +74,10 @@ struct FwdChunkParams {
   float* sa;
   bf16_t* y;
   float* sT;
-  int T, H, C;
+  int T, H;
+  int cps;                   // chunks per workgroup: all of a sequence's, or a segment's
+  const float* bound;        // segment g > 0 of [B,H,G,64,64]: its start state
+  int* fault;                // [B,H,G] (segmented calls only)
   uint32_t spin_limit;       // polls per hand-over wait (> 0)
 };
 
@@ -282,7 +285,8 @@ __device__ __forceinline__ uint4 load_stream(const uint4* q) {
   return make_uint4(x[0], x[1], x[2], x[3]);
 }
 
-template <bool kHasS0>
+// Grid (H, B, G): workgroup (h, b, g) runs segment g of the sequence, chunks
+// g cps .. (a sequence in one piece is its only segment).
 __global__ __launch_bounds__(kBlock, 1) void wkv7_fwd_chunk_kernel(const FwdChunkParams p) {
   __shared__ ChunkOps ops[kSlots];
   __shared__ __attribute__((aligned(16))) PrepLds prep[kSlots];
@@ -293,8 +297,12 @@ __global__ __launch_bounds__(kBlock, 1) void wkv7_fwd_chunk_kernel(const FwdChun
   const int h = blockIdx.x, b = blockIdx.y, H = p.H, T = p.T;
   const int64_t bh = (int64_t)b * H + h;
   const int64_t tstride = (int64_t)H * kHead;              // elements per step
-  const int64_t tok0 = ((int64_t)b * T * H + h) * kHead;   // step 0 of (b, h)
-  const int nchunks = T / kL;
+  const int g = blockIdx.z, total = T / kL;
+  const int c0 = g * p.cps, nchunks = min(p.cps, total - c0);   // this segment's chunks
+  // step 0 of (b, h)'s segment
+  const int64_t tok0 = (((int64_t)b * T + (int64_t)kL * c0) * H + h) * kHead;
+  const float* const s0 = g > 0 ? p.bound + (bh * gridDim.z + g) * (kHead * kHead)
+                        : p.s0 ? p.s0 + bh * (kHead * kHead) : nullptr;
 
   if (tid < kSlots) flags.ready[tid] = -1;
   if (tid == 0) flags.fault = 0;
@@ -346,8 +354,8 @@ __global__ __launch_bounds__(kBlock, 1) void wkv7_fwd_chunk_kernel(const FwdChun
     f32x4 S[4];
 #pragma unroll
     for (int ib = 0; ib < 4; ++ib) {
-      if (kHasS0)
-        S[ib] = *reinterpret_cast<const f32x4*>(p.s0 + bh * (kHead * kHead) + jcol * kHead + 16 * ib + 4 * qd);
+      if (s0)
+        S[ib] = *reinterpret_cast<const f32x4*>(s0 + jcol * kHead + 16 * ib + 4 * qd);
       else
         S[ib] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
@@ -358,7 +366,7 @@ __global__ __launch_bounds__(kBlock, 1) void wkv7_fwd_chunk_kernel(const FwdChun
     // the checkpoint after chunk c (chunk_len is 16 here: one per chunk),
     // transposed ([key][value]): rows = keys 16 ib + 4 qd + r, column jcol
     auto store_ckpt = [&](int c, const f32x4 (&st)[4]) {
-      float* const ck = p.ckpt + (bh * nchunks + c) * (kHead * kHead);
+      float* const ck = p.ckpt + (bh * total + c0 + c) * (kHead * kHead);
 #pragma unroll
       for (int ib = 0; ib < 4; ++ib)
 #pragma unroll
@@ -409,7 +417,7 @@ __global__ __launch_bounds__(kBlock, 1) void wkv7_fwd_chunk_kernel(const FwdChun
     }
     if (nchunks > 0) store_ckpt(nchunks - 1, S);
 
-    if (p.sT) {
+    if (p.sT && c0 + nchunks == total) {
 #pragma unroll
       for (int ib = 0; ib < 4; ++ib)
         *reinterpret_cast<f32x4*>(p.sT + bh * (kHead * kHead) + jcol * kHead + 16 * ib + 4 * qd) = S[ib];
@@ -418,19 +426,13 @@ __global__ __launch_bounds__(kBlock, 1) void wkv7_fwd_chunk_kernel(const FwdChun
 
   // every wave ends here: if any wave gave up a wait, the whole (batch,
   // head)'s outputs are unreliable, so they are overwritten with NaN and the
-  // event is counted for the host
+  // event is counted for the host; a segment leaves its word for the kernel
+  // that does this after all segments
   __syncthreads();
-  if (lds_load_flag(&flags.fault)) {
-    const float nan = __builtin_nanf("");
-    for (int64_t i = tid; i < (int64_t)T * kHead; i += kBlock) {
-      const int64_t off = tok0 + (i >> 6) * tstride + (i & 63);
-      p.y[off] = 0x7fc0;
-      p.sa[off] = nan;
-    }
-    float* const ck = p.ckpt + bh * nchunks * (kHead * kHead);
-    for (int64_t i = tid; i < (int64_t)nchunks * kHead * kHead; i += kBlock) ck[i] = nan;
-    if (p.sT)
-      for (int i = tid; i < kHead * kHead; i += kBlock) p.sT[bh * (kHead * kHead) + i] = nan;
+  if (p.fault) {
+    if (tid == 0 && lds_load_flag(&flags.fault)) p.fault[bh * gridDim.z + g] = 1;
+  } else if (lds_load_flag(&flags.fault)) {
+    poison_forward(p.y, p.sa, p.ckpt, p.sT, b, h, H, T, total, tid, kBlock);
     if (tid == 0) atomicAdd(&handover_faults, 1u);
   }
 }
@@ -469,14 +471,16 @@ hipError_t launch_forward_chunked(const ForwardDesc& d, hipStream_t stream) {
   p.sT = d.sT;
   p.T = d.T;
   p.H = d.H;
-  p.C = d.C;
+  p.cps = d.seg.G > 1 ? d.seg.cps : d.T / kL;
+  p.bound = d.seg.bound;
+  p.fault = d.seg.G > 1 ? d.seg.fault : nullptr;
   p.spin_limit = d.kc.spin_limit ? d.kc.spin_limit : kSpinLimit;
-  const dim3 grid(d.H, d.B, 1), block(kBlock, 1, 1);
-  if (d.s0)
-    hipLaunchKernelGGL(wkv7_fwd_chunk_kernel<true>, grid, block, 0, stream, p);
-  else
-    hipLaunchKernelGGL(wkv7_fwd_chunk_kernel<false>, grid, block, 0, stream, p);
-  return hipGetLastError();
+  const dim3 grid(d.H, d.B, d.seg.G), block(kBlock, 1, 1);
+  if (d.seg.G > 1)
+    if (hipError_t e = launch_segment_bounds(d, stream)) return e;
+  hipLaunchKernelGGL(wkv7_fwd_chunk_kernel, grid, block, 0, stream, p);
+  hipError_t e = hipGetLastError();
+  return e == hipSuccess && d.seg.G > 1 ? launch_segment_poison(d, stream) : e;
 }
 
 hipError_t handover_fault_counter(unsigned int** counter) {

@@ -17,6 +17,17 @@ struct KernelChoice {
   uint32_t spin_limit = 0;      // 0 = default
 };
 
+// A sequence cut into G segments of cps 16-step chunks (the last may hold
+// fewer) that run side by side (wkv7_segment.hip); G = 1: in one piece. The
+// buffers lie in the caller's workspace.
+struct Segments {
+  int G = 1, cps = 0;
+  float* bound = nullptr;       // [B,H,G,64,64]: segment g's start state (forward, g >= 1) or the
+                                // state gradient at its end (backward, g <= G - 2)
+  float* trans = nullptr;       // [B,H,G,64,64]: segment g's transition matrix
+  int* fault = nullptr;         // [B,H,G]: a hand-over wait of segment g was given up
+};
+
 // Forward pass, mirrors wkv7_forward_impl (wkv7_common/host.rs:29-183).
 struct ForwardDesc {
   Dtype dtype;
@@ -28,6 +39,7 @@ struct ForwardDesc {
   void* y;                      // [B,T,H,64] in dtype
   float* sT;                    // [B,H,64,64] or nullptr
   KernelChoice kc;
+  Segments seg;
 };
 
 // Backward pass, mirrors wkv7_backward_impl (wkv7_common/host.rs:185-369).
@@ -42,6 +54,7 @@ struct BackwardDesc {
   void *dw, *dr, *dk, *dv, *da, *db;   // [B,T,H,64] in dtype
   float* ds0;                   // [B,H,64,64] or nullptr
   KernelChoice kc;
+  Segments seg;
 };
 
 // Slot-mapped inference, mirrors wkv7_infer_forward_impl
@@ -60,6 +73,21 @@ struct InferDesc {
 };
 
 hipError_t launch_forward(const ForwardDesc& d, hipStream_t stream);
+
+// How launch_forward / launch_backward would cut this call (its shape, dtype
+// and kernel choice; the buffers are not looked at), the workspace that takes,
+// and the buffers' places in it (wkv7_segment.hip).
+Segments plan_segments(const ForwardDesc& d);
+Segments plan_segments(const BackwardDesc& d);
+int64_t segment_bytes(const Segments& s, int B, int H);
+void place_segments(Segments* s, int B, int H, void* workspace);
+// the boundary states of a call's segments, into seg.bound, and the segments'
+// fault words
+hipError_t launch_segment_bounds(const ForwardDesc& d, hipStream_t stream);
+hipError_t launch_segment_bounds(const BackwardDesc& d, hipStream_t stream);
+// after a segmented forward: every output of a (batch, head) any of whose
+// segments gave up a wait becomes NaN, and the event is counted once
+hipError_t launch_segment_poison(const ForwardDesc& d, hipStream_t stream);
 
 // Chunked matrix-core forward (wkv7_chunk_forward.hip): bf16 operands,
 // chunk_len 16. launch_forward picks it when supported, unless the caller

@@ -194,6 +194,17 @@ def _options(kernels: str = "auto", handover_spin_limit: int = 0):
     return _native.Wkv7Options(codes[kernels], int(handover_spin_limit))
 
 
+def _workspace(query: str, B, T, H, N, chunk_len, dtype, options, dev):
+    """The workspace a call is cut into segments with (include/wkv7_segments.h),
+    as (tensor or None, bytes). Allocated per call on the current stream: the
+    caching allocator hands the same block out again."""
+    nbytes = getattr(_native.lib(), query)(B, T, H, N, chunk_len, dtype,
+                                           _native.options_ref(options))
+    if nbytes <= 0:
+        return None, 0
+    return torch.empty(nbytes, dtype=torch.uint8, device=dev), nbytes
+
+
 def _forward(w, r, k, v, a, b, initial_state, chunk_len, use_initial_state, return_final_state,
              options=None):
     w, r, k, v, a, b = _tokens(w, r, k, v, a, b)
@@ -206,11 +217,14 @@ def _forward(w, r, k, v, a, b, initial_state, chunk_len, use_initial_state, retu
     output = torch.empty_like(w)
     final_state = (torch.empty((B, H, N, N), dtype=torch.float32, device=dev)
                    if return_final_state else None)
+    ws, nbytes = _workspace("wkv7_forward_workspace_bytes", B, T, H, N, chunk_len,
+                            _dtype_code(w), options, dev)
     end = _mark("forward", dev)
-    _native.call("wkv7_forward_ex", _ptr(w), _ptr(r), _ptr(k), _ptr(v), _ptr(a), _ptr(b),
+    _native.call("wkv7_forward_ws", _ptr(w), _ptr(r), _ptr(k), _ptr(v), _ptr(a), _ptr(b),
                  _ptr(s0), B, T, H, N, chunk_len, _dtype_code(w), int(use_initial_state),
                  int(return_final_state), _ptr(state), _ptr(removal_state), _ptr(output),
-                 _ptr(final_state), _native.options_ref(options), _stream(dev))
+                 _ptr(final_state), _native.options_ref(options), _ptr(ws), nbytes,
+                 _stream(dev))
     _close(end, dev)
     return state, removal_state, output, final_state
 
@@ -227,12 +241,14 @@ def _backward(w, r, k, v, a, b, state, removal_state, output_grad, final_state_g
     grads = [torch.empty_like(w) for _ in range(6)]
     ds0 = (torch.empty((B, H, N, N), dtype=torch.float32, device=dev)
            if write_initial_state_grad else None)
+    ws, nbytes = _workspace("wkv7_backward_workspace_bytes", B, T, H, N, chunk_len,
+                            _dtype_code(w), options, dev)
     end = _mark("backward", dev)
-    _native.call("wkv7_backward_ex", _ptr(w), _ptr(r), _ptr(k), _ptr(v), _ptr(a), _ptr(b),
+    _native.call("wkv7_backward_ws", _ptr(w), _ptr(r), _ptr(k), _ptr(v), _ptr(a), _ptr(b),
                  _ptr(state), _ptr(removal_state), _ptr(output_grad), _ptr(dsT),
                  B, T, H, N, chunk_len, _dtype_code(w), int(use_final_state_grad),
                  int(write_initial_state_grad), *(_ptr(g) for g in grads), _ptr(ds0),
-                 _native.options_ref(options), _stream(dev))
+                 _native.options_ref(options), _ptr(ws), nbytes, _stream(dev))
     _close(end, dev)
     return grads, ds0
 
