@@ -102,6 +102,12 @@ template <> struct Io<bf16_t> {
 __device__ __forceinline__ float sigmoid_f(float x) { return 1.0f / (1.0f + expf(-x)); }
 __device__ __forceinline__ float decay_f(float sig) { return expf(kWScale * sig); }
 
+// the decode's dither of step `seed`, wkv7_infer/kernel.rs:8-13
+__device__ __forceinline__ float dither_f(uint32_t seed) {
+  const uint32_t mixed = seed * 2654435769u;          // wrapping u32 product
+  return (float)(int32_t)mixed * 4.547473508864641e-13f;   // 2^-41
+}
+
 // ------------------------------------------------------- cross-lane reduction
 // DPP move feeding an add (the compiler fuses the pair into v_add_f32_dpp)
 template <int CTRL>

@@ -18,7 +18,9 @@
 //   is formed in fp32, gets the dither, and is rounded to bf16 once
 //   (kernel.rs:71-78); the removal-state sum, the state update and the output
 //   sum round each operation to bf16 in the kernel's order (kernel.rs:81-98),
-//   summing over the key index left to right.
+//   summing over the key index left to right. Calls of several steps on few
+//   (row, head) pairs run in wkv7_infer_prompt.hip instead, with the same
+//   results.
 //
 // Design of the fp32-state kernel: the forward kernel's thread layout and
 // per-step arithmetic (one workgroup per (active row, head), a 2x4 state
@@ -36,11 +38,6 @@ namespace {
 // bound by the HBM latency of its state read, so workgroups in flight count).
 enum { V_W = 0, V_R, V_K, V_V, V_A, V_B, V_COUNT };
 
-
-__device__ __forceinline__ float dither_f(uint32_t seed) {
-  const uint32_t mixed = seed * 2654435769u;          // wrapping u32 product
-  return (float)(int32_t)mixed * 4.547473508864641e-13f;   // 2^-41
-}
 
 template <typename Tin>
 struct InferParams {
@@ -583,6 +580,7 @@ hipError_t launch_infer_t(const InferDesc& d, hipStream_t stream) {
 
 hipError_t launch_infer(const InferDesc& d, hipStream_t stream) {
   if (d.Ba == 0 || d.H == 0) return hipSuccess;
+  if (infer_prompt_preferred(d)) return launch_infer_prompt(d, stream);
   if (d.state_dtype == Dtype::BF16) return launch_infer_bf16(d, stream);
   return d.dtype == Dtype::BF16 ? launch_infer_t<bf16_t>(d, stream) : launch_infer_t<float>(d, stream);
 }

@@ -120,6 +120,10 @@ bool chunk_f32_backward_preferred(const BackwardDesc& d);
 hipError_t launch_backward_chunked_f32(const BackwardDesc& d, hipStream_t stream);
 hipError_t launch_backward(const BackwardDesc& d, hipStream_t stream);
 hipError_t launch_infer(const InferDesc& d, hipStream_t stream);
+// bf16-state calls of several steps on few (row, head) pairs
+// (wkv7_infer_prompt.hip); launch_infer picks it where it is preferred
+bool infer_prompt_preferred(const InferDesc& d);
+hipError_t launch_infer_prompt(const InferDesc& d, hipStream_t stream);
 
 // Device self-test of the bf16 split and rounded sum (wkv7_selftest.hip);
 // n <= 2^31 * 256 pairs, pointers checked by the ABI layer.

@@ -1,0 +1,71 @@
+"""bf16-state prompts on few (row, head) pairs (wkv7_infer_prompt.hip) against
+the bf16 oracle, whose operations round in the same order: equal bit for bit,
+outputs and states, at the sizes where the staged steps and the pipelined sums
+begin and end."""
+
+import numpy as np
+import pytest
+import torch
+
+from conftest import NAMES, announce, load_pkg, to_dev, to_np
+
+pytestmark = pytest.mark.gpu
+
+
+def _mask(kind, rows, T, rng):
+    m = np.ones((rows, T), np.float32)
+    if kind == "left":                       # padding of unequal length
+        for i in range(rows):
+            m[i, :(i * 7 + 3) % T] = 0
+    elif kind == "holes":
+        m = (rng.random((rows, T)) < 0.6).astype(np.float32)
+    elif kind == "edges":                    # first row dead, then one live step each
+        m[:] = 0
+        for i in range(1, rows):
+            m[i, (T - 1) * (i % 2)] = 1
+    return m
+
+
+@pytest.mark.parametrize("rows,T,H,mask", [
+    (1, 2, 1, None), (2, 3, 2, None), (1, 4, 3, "holes"), (3, 5, 2, "edges"), (2, 8, 1, "left"),
+    (3, 63, 2, "holes"), (2, 64, 3, "left"), (3, 65, 1, "edges"), (2, 130, 2, "left"),
+    (3, 200, 2, "holes"),
+    # 128 and 129 pairs (rows of a pair over two workgroups, over one), 512 and
+    # 513 (the last that runs here, the first that does not)
+    (32, 4, 4, "holes"), (43, 4, 3, None), (43, 9, 3, "left"), (128, 4, 4, "left"), (171, 3, 3, "holes"),
+])
+def test_prompts_equal_the_oracle(oracle, rows, T, H, mask):
+    announce("bf16 prompt", rows, T, H, mask)
+    pkg = load_pkg()
+    wk = pkg.wkv7
+    rng = np.random.default_rng(rows * 1000 + T)
+    d = pkg.synthetic.make_inputs(rows, T, H, 64, seed=T, bf16=True, with_grad=False)
+    slots = rows + 2
+    state = pkg.synthetic.bf16_round(rng.standard_normal((slots, H, 64, 64)).astype(np.float32))
+    ids = rng.permutation(slots)[:rows].astype(np.int32)
+    elapsed = rng.integers(0, 5000, slots).astype(np.int32)
+    m = _mask(mask, rows, T, rng) if mask else None
+    st_gpu = to_dev(state, torch.bfloat16)
+    y = wk.wkv7_infer_forward(*(to_dev(d[n], torch.bfloat16) for n in NAMES),
+                              torch.from_numpy(ids).cuda(), st_gpu,
+                              None if m is None else to_dev(m, torch.bfloat16),
+                              torch.from_numpy(elapsed).cuda()).output
+    torch.cuda.synchronize()
+    want = state.copy()
+    y_want = oracle.infer_bf16(*(d[n] for n in NAMES), ids, want, m, elapsed.view(np.uint32))
+    assert np.array_equal(to_np(y), y_want)
+    assert np.array_equal(to_np(st_gpu), want)
+
+
+def test_a_refused_slot_touches_nothing(oracle):
+    announce("bf16 prompt, a slot out of range")
+    pkg = load_pkg()
+    d = pkg.synthetic.make_inputs(2, 6, 2, 64, seed=3, bf16=True, with_grad=False)
+    st = torch.randn(2, 2, 64, 64, device="cuda").to(torch.bfloat16)
+    before = st.clone()
+    out = pkg.wkv7.wkv7_infer_forward(*(to_dev(d[n], torch.bfloat16) for n in NAMES),
+                                      torch.tensor([7, 1], dtype=torch.int32, device="cuda"), st,
+                                      None, torch.zeros(2, dtype=torch.int32, device="cuda"))
+    torch.cuda.synchronize()
+    assert not out.output[0].any() and out.output[1].any()
+    assert torch.equal(st[0], before[0]) and not torch.equal(st[1], before[1])
