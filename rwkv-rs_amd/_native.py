@@ -32,6 +32,20 @@ class Wkv7Options(ctypes.Structure):
     _fields_ = [("kernels", ctypes.c_int), ("handover_spin_limit", ctypes.c_uint32)]
 
 
+class DecodeCellParams(ctypes.Structure):
+    """struct rwkv_decode_cell_params (include/rwkv_decode.h)."""
+    _fields_ = ([(n, ctypes.c_void_p) for n in (
+        "norm_time_weight", "norm_time_bias", "norm_channel_weight", "norm_channel_bias")]
+        + [("mix", ctypes.c_void_p * 6)]
+        + [(n, ctypes.c_void_p) for n in (
+            "receptance", "key", "value", "output", "decay_a", "decay_b", "decay_bias", "rate_a",
+            "rate_b", "rate_bias", "residual_a", "residual_b", "residual_bias", "gate_a", "gate_b",
+            "key_removal", "key_replacement", "bonus", "group_norm_weight", "group_norm_bias",
+            "channel_mix", "channel_key", "channel_value")]
+        + [(n, ctypes.c_int64) for n in ("decay_rank", "rate_rank", "residual_rank", "gate_rank")]
+        + [(n, ctypes.c_float) for n in ("norm_time_eps", "norm_channel_eps", "group_norm_eps")])
+
+
 def options_ref(opts):
     """A pointer argument for an optional wkv7_options (None -> NULL)."""
     return None if opts is None else ctypes.cast(ctypes.pointer(opts), ctypes.c_void_p)
@@ -56,6 +70,9 @@ EXPORTS = (
 # and those of include/wkv7_segments.h
 SEGMENT_EXPORTS = ("wkv7_forward_workspace_bytes", "wkv7_backward_workspace_bytes",
                    "wkv7_forward_ws", "wkv7_backward_ws")
+
+# and of include/rwkv_decode.h
+DECODE_EXPORTS = ("rwkv_decode_workspace_bytes", "rwkv_decode_cell", "rwkv_decode_head")
 
 _P = ctypes.c_void_p
 _I64 = ctypes.c_int64
@@ -98,6 +115,9 @@ _SIGNATURES = {
     "rwkv_weight_prepare_forward": ([_P] * 11 + [_I64] * 3 + [_INT] * 2 + [_P] * 6, _INT),
     "rwkv_weight_prepare_backward": ([_P] * 11 + [_I64] * 3 + [_INT] * 2 + [_P] * 17
                                      + [_I64, _P], _INT),
+    "rwkv_decode_workspace_bytes": ([_I64] * 2, _I64),
+    "rwkv_decode_cell": ([_P] * 9 + [_I64] * 3 + [_INT] * 2 + [_P, _I64, _P], _INT),
+    "rwkv_decode_head": ([_P] * 3 + [ctypes.c_float, _P] + [_I64] * 3 + [_P] * 2 + [_I64, _P], _INT),
     "rwkv_cross_entropy_l2wrap_forward": ([_P] * 2 + [_I64] * 2 + [_INT] + [_P] * 5, _INT),
     "rwkv_cross_entropy_l2wrap_backward": ([_P] * 6 + [ctypes.c_float] + [_I64] * 2 + [_INT]
                                            + [_P] * 2, _INT),

@@ -41,6 +41,7 @@
 #include <mutex>
 #include <type_traits>
 
+#include "neighbors_device.hpp"
 #include "neighbors_launch.hpp"
 
 namespace rwkv_nb {
@@ -853,15 +854,6 @@ __global__ __launch_bounds__(256) void readout_backward_kernel(ReadoutArgs a) {
 }
 
 // ------------------------------------------------- weight preparation, end
-constexpr float kNormEps = 1e-12f;       // F.normalize's eps (weight_prepare.rs:313)
-constexpr float kSoftplusLinear = 20.f;  // softplus(y) = y above this, as torch's
-
-__device__ __forceinline__ float sigmoid1(float x) { return 1.f / (1.f + expf(-x)); }
-
-__device__ __forceinline__ float softplus1(float y) {
-  return y > kSoftplusLinear ? y : log1pf(expf(y));
-}
-
 // softplus'(y)
 __device__ __forceinline__ float softplus_slope(float y) {
   return y > kSoftplusLinear ? 1.f : sigmoid1(y);

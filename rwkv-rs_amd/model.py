@@ -47,6 +47,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from . import decode as _decode
 from . import lm_loss as _loss
 from . import neighbors as _nb
 from . import wkv7 as _wkv7
@@ -613,7 +614,9 @@ class AutoRegressiveModel(nn.Module):
         with ``infer_state.elapsed_t`` as the dither's step count (the
         caller advances it afterwards, ``InferState.advance``, as
         inferring.rs:276 does). ``context_mask`` ([batch, T], 0/1) marks
-        valid steps; a masked step leaves its slot's state alone. Returns
+        valid steps; a masked step leaves its slot's state alone. A step of
+        one token runs on the fused kernels of ``decode`` where they take it
+        (bf16 autocast, fp32 parameters, no mask). Returns
         the logits of the last step ([batch, 1, vocab], "last"), of every
         step ("full") or None ("skip")."""
         if unembed_mode not in UNEMBED_MODES:
@@ -621,6 +624,9 @@ class AutoRegressiveModel(nn.Module):
         B, T = contexts.shape
         if T == 0:
             raise ValueError("contexts must be non-empty")
+        fused = _decode.step(self, contexts, batch_ids, infer_state, context_mask, unembed_mode)
+        if fused is not None:
+            return fused[0]
         kernel = _wkv7.KernelInfer
         x = self.layer_norm_for_first_cell(self.embed(contexts))
         x, st, state, sc = self.cells(x, batch_ids, kernel, infer_state.elapsed_t, context_mask,

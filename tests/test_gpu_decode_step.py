@@ -1,0 +1,118 @@
+"""One decode step of the model on the fused kernels (include/rwkv_decode.h)
+against the modules it stands in for, at the sizes where its row tiles, column
+tiles and slots begin and end. Both round every intermediate to bf16 at the same
+places and differ only in the order of sums, so a value near a tie comes out one
+bf16 ulp off and travels on: per layer about 3e-3 relative, held to 1e-2 on a
+two-cell model's logits and shifts."""
+
+import pytest
+import torch
+
+from conftest import announce, load_pkg
+from model_helpers import tiny_model
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _err(a, b):
+    a, b = a.double(), b.double()
+    return float((a - b).norm() / b.norm())
+
+
+def _model(heads=2, vocab=97, cells=2, seed=1):
+    return tiny_model(seed=seed, cells=cells, heads=heads, vocab=vocab, std=0.2,
+                      wkv7_dtype=torch.bfloat16, neighbor_ops="hip").to(DEV)
+
+
+def _state(model, slots, state_dtype, seed):
+    g = torch.Generator(DEV).manual_seed(seed)
+    st = model.new_infer_state(slots, state_dtype=state_dtype)
+    for t in st.shift_time + st.state + st.shift_channel:
+        t.copy_(torch.randn(t.shape, generator=g, device=DEV) * 0.5)
+    st.elapsed_t.copy_(torch.randint(0, 99, (slots,), generator=g, device=DEV))
+    return st
+
+
+def _infer(model, toks, ids, st, mode="last"):
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        return model.infer(toks, ids, st, unembed_mode=mode)
+
+
+@pytest.mark.parametrize("rows,slots,heads,vocab,state_dtype", [
+    (1, 1, 1, 1, torch.bfloat16), (3, 5, 2, 97, torch.bfloat16), (16, 16, 2, 16, torch.float32),
+    (17, 20, 3, 33, torch.bfloat16), (33, 33, 2, 97, torch.float32), (64, 70, 2, 130, torch.bfloat16),
+])
+def test_a_fused_step_matches_the_modules(monkeypatch, rows, slots, heads, vocab, state_dtype):
+    announce("decode step", rows, slots, heads, vocab, str(state_dtype))
+    decode = load_pkg().decode
+    model = _model(heads, vocab)
+    ids = torch.randperm(slots, generator=torch.Generator().manual_seed(rows))[:rows].to(DEV)
+    toks = torch.randint(0, vocab, (rows, 1), generator=torch.Generator().manual_seed(3)).to(DEV)
+    a, b = _state(model, slots, state_dtype, 7), _state(model, slots, state_dtype, 7)
+    before = [t.clone() for t in a.state + a.shift_time + a.shift_channel]
+    taken = []
+    real = decode.step
+    monkeypatch.setattr(decode, "step", lambda *x: taken.append(real(*x)) or taken[-1])
+    got = _infer(model, toks, ids, a)
+    monkeypatch.setattr(decode, "step", lambda *x: None)
+    want = _infer(model, toks, ids, b)
+    torch.cuda.synchronize()
+    assert taken[0] is not None and got.dtype == want.dtype and got.shape == want.shape
+    assert _err(got, want) < 1e-2
+    idle = [s for s in range(slots) if s not in ids.tolist()]
+    for x, y, z in zip(a.state + a.shift_time + a.shift_channel,
+                       b.state + b.shift_time + b.shift_channel, before):
+        assert x.dtype == y.dtype and _err(x, y) < 1e-2
+        assert torch.equal(x[idle], z[idle])
+    monkeypatch.setattr(decode, "step", real)
+    c = _state(model, slots, state_dtype, 7)
+    assert _infer(model, toks, ids, c, "skip") is None
+    assert all(torch.equal(x, y) for x, y in zip(c.state + c.shift_time, a.state + a.shift_time))
+
+
+def test_what_the_kernels_do_not_take_goes_through_the_modules():
+    announce("decode step, calls that stay with the modules")
+    decode = load_pkg().decode
+    model = _model()
+    st = _state(model, 4, torch.bfloat16, 1)
+    ids, toks = torch.arange(3, device=DEV), torch.zeros(3, 1, dtype=torch.long, device=DEV)
+
+    def taken(m=model, t=toks, i=ids, s=st, mask=None):
+        with torch.autocast("cuda", dtype=torch.bfloat16), torch.no_grad():
+            return decode.step(m, t, i, s, mask, "last") is not None
+    assert taken()
+    assert not taken(t=toks.expand(3, 2)) and not taken(mask=torch.ones(3, 1, device=DEV))
+    with torch.no_grad():
+        assert decode.step(model, toks, ids, st, None, "last") is None      # no autocast
+    seen = []
+    hook = model.cells.cells[1].channel_mixer.key.register_forward_hook(lambda *x: seen.append(1))
+    assert not taken()
+    _infer(model, toks, ids, st)
+    assert seen == [1]
+    hook.remove()
+    assert taken()
+
+    class Other(torch.nn.Linear):
+        pass
+    old = model.cells.cells[0].time_mixer.gated_readout.projection_output
+    model.cells.cells[0].time_mixer.gated_readout.projection_output = Other(128, 128, bias=False).to(DEV)
+    assert not taken()
+    model.cells.cells[0].time_mixer.gated_readout.projection_output = old
+    w = model.cells.cells[0].channel_mixer.key.weight
+    w.data = w.data.t().contiguous().t()
+    assert not taken()
+    w.data = w.data.contiguous().to(torch.bfloat16)
+    assert not taken()
+
+
+def test_an_id_out_of_range_touches_no_slot():
+    announce("decode step, a slot out of range")
+    model = _model()
+    st, ref = _state(model, 4, torch.bfloat16, 2), _state(model, 4, torch.bfloat16, 2)
+    toks = torch.arange(2, device=DEV).reshape(2, 1)
+    _infer(model, toks, torch.tensor([9, 2], device=DEV), st)
+    torch.cuda.synchronize()
+    for x, y in zip(st.state + st.shift_time + st.shift_channel,
+                    ref.state + ref.shift_time + ref.shift_channel):
+        assert torch.equal(x[[0, 1, 3]], y[[0, 1, 3]]) and not torch.equal(x[2], y[2])
