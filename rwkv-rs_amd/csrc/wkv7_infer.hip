@@ -176,6 +176,150 @@ __global__ __launch_bounds__(kThreads) void wkv7_infer_kernel(InferParams<Tin> p
   __builtin_nontemporal_store(nt4s{St[0], St[1], St[2], St[3]}, reinterpret_cast<nt4s*>(st + rt * kHead));
 }
 
+// The same steps for several steps on few (row, head) pairs, where the 2x4
+// block's instructions bound the step: about 60 a wave, and a wave issues one
+// every 6-8 cycles while its SIMD has at most two. Here a thread holds one row
+// and four columns, half the instructions, and a pair's rows go to two
+// workgroups of eight such waves; four more waves of each stage the next tile's
+// operands (the decays' exponentials among them) and write the last one's
+// outputs beside them. Sums run in the same order, so the results are the same
+// bit for bit. T = 256, us, the kernel above and this one: 12 pairs 74 / 46, 64
+// pairs 76 / 48, 128 pairs 76 / 50, 256 pairs 82 / 78, 512 pairs 116 / 139. Four
+// workgroups of 16 rows took the same time up to 128 pairs; without the staging
+// waves, whose work the eight then share, 54 us at 36 pairs.
+constexpr int kRows = 32;
+constexpr int kRowsBlock = 16 * kRows + 256;
+template <typename Tin>
+__global__ __launch_bounds__(kRowsBlock) void wkv7_infer_rows_kernel(InferParams<Tin> p) {
+  constexpr int kTile = 16;
+  __shared__ float4 tile[2][V_COUNT][kTile + 1][16];   // a row past the last: read ahead, not used
+  __shared__ float ost[2][kTile][kRows];
+  __shared__ int live[2][kTile];
+
+  const int h = blockIdx.x, bi = blockIdx.y, j0 = kRows * blockIdx.z;
+  const bool stager = __builtin_amdgcn_readfirstlane(threadIdx.x / (16 * kRows)) != 0;
+  const int tid = stager ? threadIdx.x - 16 * kRows : threadIdx.x;
+  const int L = tid & 15, row = tid >> 4;   // columns 4L.., value row j0 + row
+  const int T = p.T;
+  const int64_t slot = p.batch_ids[bi];
+  const int64_t tstride = (int64_t)p.H * kHead;
+  const int64_t tok0 = ((int64_t)bi * T * p.H + h) * kHead;
+  if (slot < 0 || slot >= p.full_batch) {   // refused: zero output, no state touched
+    for (int64_t i = threadIdx.x; i < (int64_t)T * kRows; i += kRowsBlock) p.y[tok0 + (i / kRows) * tstride + j0 + i % kRows] = Tin(0);
+    return;
+  }
+  const int ntiles = (T + kTile - 1) / kTile;
+  typedef Io<Tin> io;
+  if (stager) {
+    const Tin* const in[V_COUNT] = {p.w, p.r, p.k, p.v, p.a, p.b};
+    typename io::raw pre[V_COUNT];
+    bool pre_live = true;
+    // thread (row, L) stages step `row` of a tile, channels 4L..
+    auto gload = [&](int ti) {
+      const int t = ti * kTile + row;
+      if (t < T) {
+        pre_live = !p.mask || mask_on<Tin>(p.mask, (int64_t)bi * T + t);
+        const int64_t off = tok0 + (int64_t)t * tstride + 4 * L;
+#pragma unroll
+        for (int i = 0; i < V_COUNT; ++i) pre[i] = io::load(in[i] + off);
+      }
+    };
+    auto lstore = [&](int ti) {
+      const bool valid = ti * kTile + row < T;
+      if (valid) {
+#pragma unroll
+        for (int i = 0; i < V_COUNT; ++i) {
+          float4 x = io::widen(pre[i]);
+          if (i == V_W) {
+            x.x = decay_f(sigmoid_f(x.x));
+            x.y = decay_f(sigmoid_f(x.y));
+            x.z = decay_f(sigmoid_f(x.z));
+            x.w = decay_f(sigmoid_f(x.w));
+          }
+          tile[ti & 1][i][row][L] = x;
+        }
+      }
+      if (L == 0) live[ti & 1][row] = valid && pre_live ? 1 : 0;
+    };
+    auto outputs = [&](int ti) {   // kRows / 4 threads a step
+      const int s = tid / (kRows / 4), c = 4 * (tid % (kRows / 4)), t = ti * kTile + s;
+      if (s < kTile && t < T)
+        io::store(p.y + tok0 + (int64_t)t * tstride + j0 + c, *reinterpret_cast<const float4*>(&ost[ti & 1][s][c]));
+    };
+    gload(0);
+    lstore(0);
+    gload(1);
+    lds_barrier();
+    for (int ti = 0; ti < ntiles; ++ti) {
+      if (ti > 0) outputs(ti - 1);
+      if (ti + 1 < ntiles) {
+        lstore(ti + 1);
+        gload(ti + 2);
+      }
+      lds_barrier();
+    }
+    outputs(ntiles - 1);
+    return;
+  }
+
+  float* const st = p.state + (slot * p.H + h) * (kHead * kHead) + (j0 + row) * kHead + 4 * L;
+  float S[4];
+  {
+    const float4 x = *reinterpret_cast<const float4*>(st);
+    S[0] = x.x; S[1] = x.y; S[2] = x.z; S[3] = x.w;
+  }
+  auto row_sum = [](float x) {   // over the 16 lanes of the row, in row_pair_sum's order
+    x += dpp_mov<kDppRor8>(x);
+    x += dpp_mov<kDppHalfMirror>(x);
+    x += dpp_mov<kDppQuadSwap2>(x);
+    x += dpp_mov<kDppQuadSwap1>(x);
+    return x;
+  };
+  lds_barrier();
+  for (int ti = 0; ti < ntiles; ++ti) {
+    const int buf = ti & 1, nst = min(kTile, T - ti * kTile);
+    uint32_t on = 0;   // the unmasked steps of the tile, one bit each
+#pragma unroll
+    for (int s = 0; s < kTile; ++s) on |= live[buf][s] ? 1u << s : 0u;
+    on = __builtin_amdgcn_readfirstlane(on);
+    // a step's operands are read during the step before it
+    struct Ops { float4 w, a, b, k, r; float v; };
+    auto read = [&](int s) {
+      return Ops{tile[buf][V_W][s][L], tile[buf][V_A][s][L], tile[buf][V_B][s][L], tile[buf][V_K][s][L],
+                 tile[buf][V_R][s][L], reinterpret_cast<const float*>(tile[buf][V_V][s])[j0 + row]};
+    };
+    auto step = [&](int s, const Ops& o) {
+      float y = 0.0f;
+      if ((on >> s) & 1) {
+        const float w[4] = {o.w.x, o.w.y, o.w.z, o.w.w}, a[4] = {o.a.x, o.a.y, o.a.z, o.a.w};
+        const float b[4] = {o.b.x, o.b.y, o.b.z, o.b.w}, k[4] = {o.k.x, o.k.y, o.k.z, o.k.w};
+        const float r[4] = {o.r.x, o.r.y, o.r.z, o.r.w};
+        float sa = a[0] * S[0];
+#pragma unroll
+        for (int c = 1; c < 4; ++c) sa = __builtin_fmaf(a[c], S[c], sa);
+        sa = row_sum(sa);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          S[c] = __builtin_fmaf(k[c], o.v, __builtin_fmaf(b[c], sa, S[c] * w[c]));
+          y = c == 0 ? r[c] * S[c] : __builtin_fmaf(r[c], S[c], y);
+        }
+        y = row_sum(y);
+      }
+      if (L == 0) ost[buf][s][row] = y;
+    };
+    Ops x = read(0), z;
+    for (int s = 0; s < nst; s += 2) {   // two steps an iteration, so that x and z need no moves
+      z = read(s + 1);
+      step(s, x);
+      if (s + 1 >= nst) break;
+      x = read(s + 2 < kTile ? s + 2 : kTile);
+      step(s + 1, z);
+    }
+    lds_barrier();
+  }
+  *reinterpret_cast<float4*>(st) = make_float4(S[0], S[1], S[2], S[3]);
+}
+
 // ------------------------------------------------------------ bf16 state
 // One wave per (active row, head); lane j owns value row j of the state, so
 // each row's sums over the key index run left to right inside one lane, as
@@ -571,6 +715,8 @@ hipError_t launch_infer_t(const InferDesc& d, hipStream_t stream) {
   const dim3 grid(d.H, d.Ba, 1), block(kThreads, 1, 1);
   if (d.T == 1)
     hipLaunchKernelGGL((wkv7_infer_kernel<Tin, 1>), grid, block, 0, stream, p);
+  else if ((int64_t)d.Ba * d.H <= 256)   // its comment has both sides' times
+    hipLaunchKernelGGL(wkv7_infer_rows_kernel<Tin>, dim3(d.H, d.Ba, kHead / kRows), dim3(kRowsBlock), 0, stream, p);
   else
     hipLaunchKernelGGL((wkv7_infer_kernel<Tin, 16>), grid, block, 0, stream, p);
   return hipGetLastError();

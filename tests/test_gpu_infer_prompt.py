@@ -1,7 +1,8 @@
-"""bf16-state prompts on few (row, head) pairs (wkv7_infer_prompt.hip) against
-the bf16 oracle, whose operations round in the same order: equal bit for bit,
-outputs and states, at the sizes where the staged steps and the pipelined sums
-begin and end."""
+"""Prompts on few (row, head) pairs. bf16 state (wkv7_infer_prompt.hip) against
+the bf16 oracle, whose operations round in the same order; fp32 state
+(wkv7_infer_rows_kernel) against the same rows in a call that is too large for
+it. Both equal bit for bit, outputs and states, at the sizes where the staged
+steps and tiles begin and end."""
 
 import numpy as np
 import pytest
@@ -69,3 +70,31 @@ def test_a_refused_slot_touches_nothing(oracle):
     torch.cuda.synchronize()
     assert not out.output[0].any() and out.output[1].any()
     assert torch.equal(st[0], before[0]) and not torch.equal(st[1], before[1])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("rows,T,H,mask", [
+    (1, 2, 1, None), (2, 15, 3, "holes"), (3, 16, 2, "left"), (2, 17, 2, None), (3, 33, 2, "edges"),
+    (64, 18, 4, "holes"),                                   # 256 pairs: the last that run here
+])
+def test_fp32_state_prompts_equal_a_larger_call(dtype, rows, T, H, mask):
+    announce("fp32-state prompt", rows, T, H, mask, str(dtype))
+    pkg = load_pkg()
+    all_rows = max(rows, 256 // H) + 1                      # over 256 pairs
+    rng = np.random.default_rng(T)
+    d = pkg.synthetic.make_inputs(all_rows, T, H, 64, seed=T + rows, bf16=dtype == torch.bfloat16,
+                                  with_grad=False)
+    ops = [to_dev(d[n], dtype) for n in NAMES]
+    m = torch.from_numpy(_mask(mask, all_rows, T, rng)).cuda().to(dtype) if mask else None
+    ids = torch.from_numpy(rng.permutation(all_rows).astype(np.int32)).cuda()
+    state = torch.from_numpy(rng.standard_normal((all_rows, H, 64, 64)).astype(np.float32)).cuda()
+    big, small = state.clone(), state.clone()
+    want = pkg.wkv7.wkv7_infer_forward(*ops, ids, big, m, None).output
+    got = pkg.wkv7.wkv7_infer_forward(*(x[:rows].contiguous() for x in ops), ids[:rows].contiguous(),
+                                      small, None if m is None else m[:rows].contiguous(), None).output
+    torch.cuda.synchronize()
+    assert torch.equal(got, want[:rows])
+    used = ids[:rows].long()
+    assert torch.equal(small[used], big[used])
+    rest = ids[rows:].long()
+    assert torch.equal(small[rest], state[rest])
