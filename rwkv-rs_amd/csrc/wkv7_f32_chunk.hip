@@ -189,6 +189,9 @@ struct F32FwdParams {
   float* sT;                  // [B,H,64,64] or null
   unsigned int* faults;       // the chunked forwards' hand-over fault counter
   int T, H, C;
+  int cps;                    // chunks per workgroup: all of a sequence's, or a segment's
+  const float* bound;         // segment g > 0 of [B,H,G,64,64]: its start state
+  int* fault;                 // [B,H,G] (segmented calls only)
   uint32_t spin_limit;        // polls per hand-over wait (> 0)
 };
 
@@ -225,7 +228,10 @@ __device__ __forceinline__ f32x4 col_frag4(const Tin* base, int64_t tstride, int
   return x;
 }
 
-template <typename Tin, bool kHasS0>
+// Grid (H, B, G): workgroup (h, b, g) runs segment g of the sequence, chunks
+// g cps .. (a sequence in one piece is its only segment); a segment is a whole
+// number of checkpoint intervals.
+template <typename Tin>
 __global__ __launch_bounds__(kBlock, 1) void wkv7_fwd_f32_chunk_kernel(const F32FwdParams<Tin> p) {
   __shared__ F32ChunkOps ops[kSlots];
   __shared__ F32PrepLds prep[kSlots];
@@ -238,8 +244,10 @@ __global__ __launch_bounds__(kBlock, 1) void wkv7_fwd_f32_chunk_kernel(const F32
   const int h = blockIdx.x, b = blockIdx.y, H = p.H, T = p.T;
   const int64_t bh = (int64_t)b * H + h;
   const int64_t tstride = (int64_t)H * kHead;
-  const int64_t tok0 = ((int64_t)b * T * H + h) * kHead;
-  const int nchunks = T / kL;
+  const int g = blockIdx.z, c0 = g * p.cps, nchunks = min(p.cps, T / kL - c0);   // this segment's chunks
+  const int64_t tok0 = (((int64_t)b * T + (int64_t)kL * c0) * H + h) * kHead;
+  const float* const s0 = g > 0 ? p.bound + (bh * gridDim.z + g) * (kHead * kHead)
+                        : p.s0 ? p.s0 + bh * (kHead * kHead) : nullptr;
   const int per_ckpt = p.C / kL;
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
 
@@ -396,14 +404,14 @@ __global__ __launch_bounds__(kBlock, 1) void wkv7_fwd_f32_chunk_kernel(const F32
 #pragma unroll
     for (int ib = 0; ib < 4; ++ib) {
       // s0 is [value][key]: register r holds key 16 ib + 4 qd + r of value jcol
-      if (kHasS0)
-        S[ib] = *reinterpret_cast<const f32x4*>(p.s0 + bh * (kHead * kHead) + jcol * kHead + 16 * ib + 4 * qd);
+      if (s0)
+        S[ib] = *reinterpret_cast<const f32x4*>(s0 + jcol * kHead + 16 * ib + 4 * qd);
       else
         S[ib] = zero;
     }
     // the checkpoint after checkpoint group n, transposed ([key][value])
     auto store_ckpt = [&](int n) {
-      float* const ck = p.ckpt + (bh * (T / p.C) + n) * (kHead * kHead);
+      float* const ck = p.ckpt + (bh * (T / p.C) + c0 / per_ckpt + n) * (kHead * kHead);
 #pragma unroll
       for (int ib = 0; ib < 4; ++ib)
 #pragma unroll
@@ -465,7 +473,7 @@ __global__ __launch_bounds__(kBlock, 1) void wkv7_fwd_f32_chunk_kernel(const F32
       }
       if ((c + 1) % per_ckpt == 0) store_ckpt((c + 1) / per_ckpt - 1);
     }
-    if (p.sT) {
+    if (p.sT && c0 + nchunks == T / kL) {
 #pragma unroll
       for (int ib = 0; ib < 4; ++ib)
         *reinterpret_cast<f32x4*>(p.sT + bh * (kHead * kHead) + jcol * kHead + 16 * ib + 4 * qd) = S[ib];
@@ -474,20 +482,220 @@ __global__ __launch_bounds__(kBlock, 1) void wkv7_fwd_f32_chunk_kernel(const F32
 
   // every wave ends here: if any wave gave up a wait, the whole (batch,
   // head)'s outputs are unreliable, so they are overwritten with NaN and the
-  // event is counted for the host
+  // event is counted for the host; a segment leaves its word for the kernel
+  // that does this after all segments
   __syncthreads();
-  if (lds_load_flag(&flags.fault)) {
-    const float nan = __builtin_nanf("");
-    for (int64_t i = tid; i < (int64_t)T * kHead; i += kBlock) {
-      const int64_t off = tok0 + (i >> 6) * tstride + (i & 63);
-      Io<Tin>::put1(&p.y[off], nan);
-      p.sa[off] = nan;
-    }
-    float* const ck = p.ckpt + bh * (T / p.C) * (kHead * kHead);
-    for (int64_t i = tid; i < (int64_t)(T / p.C) * kHead * kHead; i += kBlock) ck[i] = nan;
-    if (p.sT)
-      for (int i = tid; i < kHead * kHead; i += kBlock) p.sT[bh * (kHead * kHead) + i] = nan;
+  if (p.fault) {
+    if (tid == 0 && lds_load_flag(&flags.fault)) p.fault[bh * gridDim.z + g] = 1;
+  } else if (lds_load_flag(&flags.fault)) {
+    poison_forward(p.y, p.sa, p.ckpt, p.sT, b, h, H, T, T / p.C, tid, kBlock);
     if (tid == 0) atomicAdd(p.faults, 1u);
+  }
+}
+
+// ---------------------------------------------- segments' transition, fp32
+// The transition of a segment (wkv7_segment.hip) with fp32 products: eight
+// prep waves, wave 4 + s preparing chunks s, s + 8, ... of the chain's order
+// into slot s % 4, and four chain waves that carry N's and M's states, as the
+// bf16 kernel does. Forward, the chain per chunk is the forward's:
+//   SA = W S^T + U,  S <- S diag(gamma_L) + V^T K- + SA^T B-,
+//   W = P A^,  U = (P A_ak) V;
+// backward it is the same form, with dY for V,
+//   dSA = W dS^T + U,  dS <- dS diag(gamma_L) + dY^T R^ + dSA^T A^,
+//   W = P^T B-,  U = (P^T A_rb^T) dY.
+// What bounds a call on few pairs is the chain, 3.1 us a chunk forward and 7.6
+// backward however many of the 256 CUs are free. B 2, H 8, T 256, fp32, back to
+// back: forward 52 us in one piece, 37 in segments (what its three launches
+// take the host); backward 128 and 41. A segmented call takes 5.7 (forward)
+// and 9.6 (backward) us per chunk of a segment.
+constexpr int kSegPrepWaves = 8;
+constexpr int kSegBlock = 64 * (kChainWaves + kSegPrepWaves);
+struct F32SegOps {
+  f32x4 w[4][64];          // W per key tile, row fragments
+  f32x4 v[4][64];          // V / dY per value tile, column fragments
+  f32x4 u[4][64];          // U per value tile, result layout
+  float f[64 * kLs];       // K- or R^, [key][step]
+  float g[64 * kLs];       // B- or A^, [key][step]
+  float gl[64];            // gamma_L
+};
+struct F32SegPrep {
+  float e[64 * kLs];       // A^ or B-, [key][step]
+  float aab[kL * kLg];     // A_ab, [t][s]
+  float aak[kL * kLg];     // A_ak, [t][s] (forward)
+};
+template <typename Tin>
+struct F32SegParams {
+  const Tin* in[5];        // x, a, b, then k and v (forward) or r and dy (backward)
+  const float* edge;
+  float *bound, *trans;
+  int* fault;
+  int T, H, G, cps;
+  uint32_t spin_limit;
+};
+
+template <typename Tin, bool kBwd>
+__global__ __launch_bounds__(kSegBlock, 1) void wkv7_transition_f32_kernel(const F32SegParams<Tin> p) {
+  __shared__ F32SegOps ops[kSlots];
+  __shared__ F32SegPrep prep[kSegPrepWaves];
+  __shared__ F32Flags flags;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int t = lane & 15, qd = lane >> 4;
+  const int h = blockIdx.x, b = blockIdx.y, H = p.H, T = p.T;
+  const int g = kBwd ? blockIdx.z + 1 : blockIdx.z;
+  const int64_t bh = (int64_t)b * H + h;
+  const int64_t tstride = (int64_t)H * kHead;
+  const int c0 = g * p.cps, n = min(p.cps, T / kL - c0);
+  const int64_t tok0 = (((int64_t)b * T + (int64_t)kL * c0) * H + h) * kHead;
+  auto chunk_of = [&](int i) { return kBwd ? n - 1 - i : i; };
+  // the segment at the known end of the sequence: N starts from the given
+  // state, and M is not needed
+  const bool edge = kBwd ? g == p.G - 1 : g == 0;
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+
+  if (tid < kSlots) flags.ready[tid] = -1;
+  if (tid == 0) flags.fault = 0;
+  if (tid < kSlots * kChainWaves) flags.taken[tid / kChainWaves][tid % kChainWaves] = tid / kChainWaves - kSlots;
+  __syncthreads();
+
+  float* const out_n = p.bound + (bh * p.G + (kBwd ? g - 1 : g + 1)) * (kHead * kHead);
+  float* const out_m = p.trans + (bh * p.G + g) * (kHead * kHead);
+  if (wave >= kChainWaves) {
+    const int s = wave - kChainWaves, slot = s % kSlots;
+    F32SegPrep& my = prep[s];
+    F32SegOps& o = ops[slot];
+    for (int i = s; i < n; i += kSegPrepWaves) {
+      const int c = chunk_of(i);
+      // the rows as fragments: x, a, b and k / r at step t, keys 16 kk + 4 qd +
+      // r; v / dy at steps 4 qd + r, values 16 vb + t
+      f32x4 X[4], A[4], B[4], F[4], V[4];
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk) {
+        X[kk] = row_frag4(p.in[0] + tok0, tstride, c, t, kk, qd);
+        A[kk] = row_frag4(p.in[1] + tok0, tstride, c, t, kk, qd);
+        B[kk] = row_frag4(p.in[2] + tok0, tstride, c, t, kk, qd);
+        F[kk] = row_frag4(p.in[3] + tok0, tstride, c, t, kk, qd);
+        V[kk] = col_frag4(p.in[4] + tok0, tstride, c, t, kk, qd);
+      }
+      f32x4 gL[4];
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float gam = gamma_of(X[kk][r]);
+          const float gin = 1.0f / gam;
+          gL[kk][r] = row_last16(gam);
+          A[kk][r] *= row_prev16(gam);          // A^
+          B[kk][r] *= gin;                      // B~
+          F[kk][r] *= kBwd ? gam : gin;         // R^ or K~
+        }
+      // row fragments of the step products: lane (qd, t) holds A_xy[t][4 qd + r]
+      f32x4 aab = zero, q = zero;
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk) {
+        aab = mm16(B[kk], A[kk], aab);
+        q = kBwd ? mm16(B[kk], F[kk], q) : mm16(F[kk], A[kk], q);   // A_rb or A_ak
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int sx = 4 * qd + r;
+        if (!(sx < t)) aab[r] = 0.f;
+        if (kBwd ? !(sx <= t) : !(sx < t)) q[r] = 0.f;
+      }
+      *reinterpret_cast<f32x4*>(&my.aab[t * kLg + 4 * qd]) = aab;
+      if (!kBwd) *reinterpret_cast<f32x4*>(&my.aak[t * kLg + 4 * qd]) = q;
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          my.e[(16 * kk + 4 * qd + r) * kLs + t] = kBwd ? B[kk][r] * gL[kk][r] : A[kk][r];
+      wave_lds_sync();
+      f32x4 P, Pt;
+      unit_lower_inverse_f32(col4(my.aab, kLg, t, qd), aab, t, qd, P, Pt);
+      // the slot is free once every chain wave has taken chunk i - 4
+      bool ok = true;
+      for (int w = 0; w < kChainWaves; ++w) ok &= wait_flag(&flags.taken[slot][w], i - kSlots, p.spin_limit);
+      if (!ok && lane == 0) lds_store_flag(&flags.fault, 1);
+      lds_acquire();
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk) {
+        o.v[kk][lane] = V[kk];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int at = (16 * kk + 4 * qd + r) * kLs + t;
+          o.f[at] = kBwd ? F[kk][r] : F[kk][r] * gL[kk][r];
+          o.g[at] = kBwd ? A[kk][r] : B[kk][r] * gL[kk][r];
+        }
+        if (t == 0) *reinterpret_cast<f32x4*>(&o.gl[16 * kk + 4 * qd]) = gL[kk];
+        // W^T tile = A^^T P^T or B-^T P: rows = keys, column = step t
+        o.w[kk][lane] = mm16(*reinterpret_cast<const f32x4*>(&my.e[(16 * kk + t) * kLs + 4 * qd]), kBwd ? P : Pt, zero);
+      }
+      // P A_ak = (A_ak^T P^T)^T and P^T A_rb^T = (A_rb P)^T as row fragments
+      const f32x4 pq = kBwd ? mm16(q, P, zero) : mm16(col4(my.aak, kLg, t, qd), Pt, zero);
+#pragma unroll
+      for (int vb = 0; vb < 4; ++vb) o.u[vb][lane] = mm16(pq, V[vb], zero);
+      lds_release();
+      if (lane == 0) lds_store_flag(&flags.ready[slot], i);
+    }
+  } else {
+    // value tile jb; key tiles in the result layout (rows = key 16 ib + 4 qd +
+    // r, column = value jcol)
+    const int jb = wave, jcol = 16 * jb + t;
+    f32x4 SN[4], SM[4];
+#pragma unroll
+    for (int ib = 0; ib < 4; ++ib) {
+      SN[ib] = edge && p.edge
+          ? *reinterpret_cast<const f32x4*>(p.edge + bh * (kHead * kHead) + jcol * kHead + 16 * ib + 4 * qd) : zero;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) SM[ib][r] = 16 * ib + 4 * qd + r == jcol ? 1.f : 0.f;
+    }
+    auto chain = [&](auto both) {
+      constexpr bool kBoth = decltype(both)::value;   // M's state too
+      for (int i = 0; i < n; ++i) {
+        const int slot = i % kSlots;
+        if (!wait_flag(&flags.ready[slot], i, p.spin_limit) && lane == 0) lds_store_flag(&flags.fault, 1);
+        lds_acquire();
+        const F32SegOps& o = ops[slot];
+        const f32x4 v = o.v[jb][lane];
+        f32x4 sn = o.u[jb][lane], sm = zero;
+#pragma unroll
+        for (int ib = 0; ib < 4; ++ib) {
+          const f32x4 w = o.w[ib][lane];
+          sn = mm16(w, SN[ib], sn);
+          if (kBoth) sm = mm16(w, SM[ib], sm);
+        }
+#pragma unroll
+        for (int ib = 0; ib < 4; ++ib) {
+          const f32x4 f = *reinterpret_cast<const f32x4*>(&o.f[(16 * ib + t) * kLs + 4 * qd]);
+          const f32x4 gg = *reinterpret_cast<const f32x4*>(&o.g[(16 * ib + t) * kLs + 4 * qd]);
+          const f32x4 gl = *reinterpret_cast<const f32x4*>(&o.gl[16 * ib + 4 * qd]);
+          SN[ib] = mm16(gg, sn, mm16(f, v, SN[ib] * gl));
+          if (kBoth) SM[ib] = mm16(gg, sm, SM[ib] * gl);
+        }
+        // every operand has been used, so its load has completed
+        __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0)
+        lds_release();
+        if (lane == 0) lds_store_flag(&flags.taken[slot][jb], i);
+      }
+    };
+    if (edge) chain(std::false_type{});
+    else chain(std::true_type{});
+#pragma unroll
+    for (int ib = 0; ib < 4; ++ib) {
+      const int at = jcol * kHead + 16 * ib + 4 * qd;
+      *reinterpret_cast<f32x4*>(out_n + at) = SN[ib];
+      if (!edge) *reinterpret_cast<f32x4*>(out_m + at) = SM[ib];
+    }
+  }
+  // as in the bf16 kernel: N of a segment whose wait was given up is NaN, and
+  // its word says so; the segment that is not run is cleared by its neighbour
+  __syncthreads();
+  const bool bad = lds_load_flag(&flags.fault) != 0;
+  if (bad)
+    for (int i = tid; i < kHead * kHead; i += kSegBlock) out_n[i] = __builtin_nanf("");
+  if (tid == 0) {
+    p.fault[bh * p.G + g] = bad ? 1 : 0;
+    if (g == (kBwd ? 1 : p.G - 2)) p.fault[bh * p.G + (kBwd ? 0 : p.G - 1)] = 0;
   }
 }
 
@@ -503,6 +711,11 @@ struct F32BwdParams {
   float* g[O_COUNT];          // gradients [B,T,H,64]
   float* ds0;                 // [B,H,64(value),64(key)] or null
   int T, H, C;
+  // segmented calls only:
+  int cps;                    // chunks per segment
+  const float* bound;         // segment g < G - 1 of [B,H,G,64,64]: the state gradient at its end
+  const int* fault;           // [B,H,G]: a boundary gradient is not there
+  unsigned int* faults;       // the device's counter of such events
 };
 
 struct F32BwdLds {
@@ -565,6 +778,10 @@ struct F32BwdLds {
 //           S0 to LDS (key waves)
 //   key-indexed gradients of key tile w: dR, dA and their part of the decay
 //           gradient (chain waves, S0 from LDS), dK, dB and theirs (key waves)
+//
+// kSeg: grid (H, B, G), workgroup (h, b, g) runs segment g of the sequence, a
+// whole number of checkpoint intervals.
+template <bool kSeg>
 __global__ __launch_bounds__(kBlock, 1) void wkv7_bwd_f32_chunk_kernel(const F32BwdParams p) {
   __shared__ F32BwdLds L;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -574,7 +791,27 @@ __global__ __launch_bounds__(kBlock, 1) void wkv7_bwd_f32_chunk_kernel(const F32
   const int64_t bh = (int64_t)b * H + h;
   const int64_t tstride = (int64_t)H * kHead;
   const int64_t tok0 = ((int64_t)b * T * H + h) * kHead;
-  const int nchunks = T / kL;
+  const int g = kSeg ? blockIdx.z : 0, G = kSeg ? gridDim.z : 1;
+  // this segment's chunks, in reverse
+  const int first = g * p.cps, last = kSeg ? min(first + p.cps, T / kL) - 1 : T / kL - 1;
+  if (kSeg) {
+    // a boundary gradient that a given-up hand-over wait left unformed: every
+    // gradient of the (batch, head) is NaN, and the event is counted
+    bool bad = false;
+    for (int i = 1; i < G; ++i) bad |= p.fault[bh * G + i] != 0;
+    if (bad) {
+      const float nan = __builtin_nanf("");
+      for (int i = tid; i < (last + 1 - first) * kL * kHead; i += kBlock) {
+        const int64_t off = tok0 + (int64_t)(kL * first + (i >> 6)) * tstride + (i & 63);
+#pragma unroll
+        for (int m = 0; m < O_COUNT; ++m) p.g[m][off] = nan;
+      }
+      if (first == 0 && tid == 0) atomicAdd(p.faults, 1u);
+      if (p.ds0 && first == 0)
+        for (int i = tid; i < kHead * kHead; i += kBlock) p.ds0[bh * (kHead * kHead) + i] = nan;
+      return;
+    }
+  }
   const int q = p.C / kL;                           // 16-step chunks per checkpoint
   const bool chain = wave < 4;
   const int wq = wave & 3;
@@ -606,11 +843,13 @@ __global__ __launch_bounds__(kBlock, 1) void wkv7_bwd_f32_chunk_kernel(const F32
   };
 
   // chain waves: dS of the chunk end, rows = key 16 ib + 4 qd + r, column = value jcol
+  const float* const dsE = kSeg && g < G - 1 ? p.bound + (bh * G + g) * (kHead * kHead)
+                         : p.dsT ? p.dsT + bh * (kHead * kHead) : nullptr;
   f32x4 dS[4];
 #pragma unroll
   for (int ib = 0; ib < 4; ++ib) {
-    if (chain && p.dsT)
-      dS[ib] = *reinterpret_cast<const f32x4*>(p.dsT + bh * (kHead * kHead) + jcol * kHead + 16 * ib + 4 * qd);
+    if (chain && dsE)
+      dS[ib] = *reinterpret_cast<const f32x4*>(dsE + jcol * kHead + 16 * ib + 4 * qd);
     else
       dS[ib] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
@@ -627,7 +866,7 @@ __global__ __launch_bounds__(kBlock, 1) void wkv7_bwd_f32_chunk_kernel(const F32
   // reversal rebuilds the earlier start state from it in place; either is
   // handed to the chain waves through LDS (S0) for the key stage.
   f32x4 Sr[4], S0[4];
-  if (!chain && nchunks > 0) load_ckpt(T / p.C - 1, Sr);   // the end state of the last chunk
+  if (!chain && last >= first) load_ckpt((last + 1) / q - 1, Sr);   // the end state of the last chunk
   // the reference's reversal of steps hi .. lo (kernel.rs:239-246), in the
   // reference's operation order: S_{t-1} = (S_t - k v - b sa) * (1 / w~)
   // Each group's own state (the chain waves' dS, the key waves' Sr and dw
@@ -690,15 +929,15 @@ __global__ __launch_bounds__(kBlock, 1) void wkv7_bwd_f32_chunk_kernel(const F32
                                   reinterpret_cast<f32x4*>(p.g[m] + cbase + off));
   };
 
-  if (nchunks > 0) fetch(nchunks - 1);
-  for (int c = nchunks - 1; c >= 0; --c) {
+  if (last >= first) fetch(last);
+  for (int c = last; c >= first; --c) {
     const bool from_ckpt = c > 0 && c % q == 0;
     if (chain) {
       stage();
     } else {
       // dw of chunk c + 1 needs the chain waves' part, written in its key
       // stage, and its a rows, which this stage replaces
-      if (c < nchunks - 1) finish_and_store(c + 1);
+      if (c < last) finish_and_store(c + 1);
       stage();
       // a checkpointed start state replaces the reversal (read after the
       // stores, waited for three phases later)
@@ -824,7 +1063,7 @@ __global__ __launch_bounds__(kBlock, 1) void wkv7_bwd_f32_chunk_kernel(const F32
     // ---- key-indexed gradients of key tile wq: rows = step 4 qd + r,
     // column = key ki. The next chunk's rows are loaded first (their
     // registers are free from here to the next stage).
-    if (c > 0) fetch(c - 1);
+    if (c > first) fetch(c - 1);
     const float gl = L.gl[ki];
     if (chain) {
       drop(Sr);
@@ -898,8 +1137,8 @@ __global__ __launch_bounds__(kBlock, 1) void wkv7_bwd_f32_chunk_kernel(const F32
     }
     lds_barrier();
   }
-  if (!chain && nchunks > 0) finish_and_store(0);
-  if (chain && p.ds0) {
+  if (!chain && last >= first) finish_and_store(first);
+  if (chain && p.ds0 && first == 0) {
 #pragma unroll
     for (int ib = 0; ib < 4; ++ib)
       *reinterpret_cast<f32x4*>(p.ds0 + bh * (kHead * kHead) + jcol * kHead + 16 * ib + 4 * qd) = dS[ib];
@@ -941,17 +1180,18 @@ static hipError_t launch_fwd_f32(const ForwardDesc& d, hipStream_t stream) {
   p.H = d.H;
   p.C = d.C;
   p.spin_limit = d.kc.spin_limit ? d.kc.spin_limit : kSpinLimit;
+  p.cps = d.seg.G > 1 ? d.seg.cps : d.T / kL;
+  p.bound = d.seg.bound;
+  p.fault = d.seg.G > 1 ? d.seg.fault : nullptr;
   // the counter lives in the bf16 forward's code object; its address is
   // looked up on the current device at every launch (a host-side lookup, no
   // stream work, so captured launches replay it as they are)
   hipError_t e = handover_fault_counter(&p.faults);
   if (e != hipSuccess) return e;
-  const dim3 grid(d.H, d.B, 1), block(kBlock, 1, 1);
-  if (d.s0)
-    hipLaunchKernelGGL((wkv7_fwd_f32_chunk_kernel<Tin, true>), grid, block, 0, stream, p);
-  else
-    hipLaunchKernelGGL((wkv7_fwd_f32_chunk_kernel<Tin, false>), grid, block, 0, stream, p);
-  return hipGetLastError();
+  if (d.seg.G > 1 && (e = launch_segment_bounds(d, stream)) != hipSuccess) return e;
+  hipLaunchKernelGGL(wkv7_fwd_f32_chunk_kernel<Tin>, dim3(d.H, d.B, d.seg.G), dim3(kBlock), 0, stream, p);
+  e = hipGetLastError();
+  return e == hipSuccess && d.seg.G > 1 ? launch_segment_poison(d, stream) : e;
 }
 
 hipError_t launch_forward_chunked_f32(const ForwardDesc& d, hipStream_t stream) {
@@ -1001,8 +1241,41 @@ hipError_t launch_backward_chunked_f32(const BackwardDesc& d, hipStream_t stream
   p.T = d.T;
   p.H = d.H;
   p.C = d.C;
-  hipLaunchKernelGGL(wkv7_bwd_f32_chunk_kernel, dim3(d.H, d.B, 1), dim3(kBlock, 1, 1), 0, stream, p);
+  p.cps = d.seg.cps;
+  p.bound = d.seg.bound;
+  p.fault = d.seg.fault;
+  p.faults = nullptr;
+  if (d.seg.G > 1) {
+    if (hipError_t e = handover_fault_counter(&p.faults)) return e;
+    if (hipError_t e = launch_segment_bounds(d, stream)) return e;
+    hipLaunchKernelGGL(wkv7_bwd_f32_chunk_kernel<true>, dim3(d.H, d.B, d.seg.G), dim3(kBlock), 0, stream, p);
+  } else {
+    hipLaunchKernelGGL(wkv7_bwd_f32_chunk_kernel<false>, dim3(d.H, d.B, 1), dim3(kBlock), 0, stream, p);
+  }
   return hipGetLastError();
+}
+
+template <typename Tin, bool kBwd>
+static hipError_t launch_transition_f32_t(const TransitionCall& c, hipStream_t stream) {
+  F32SegParams<Tin> p;
+  for (int i = 0; i < 5; ++i) p.in[i] = static_cast<const Tin*>(c.in[i]);
+  p.edge = c.edge;
+  p.bound = c.seg.bound;
+  p.trans = c.seg.trans;
+  p.fault = c.seg.fault;
+  p.T = c.T;
+  p.H = c.H;
+  p.G = c.seg.G;
+  p.cps = c.seg.cps;
+  p.spin_limit = c.spin_limit;
+  hipLaunchKernelGGL((wkv7_transition_f32_kernel<Tin, kBwd>), dim3(c.H, c.B, p.G - 1), dim3(kSegBlock), 0, stream, p);
+  return hipGetLastError();
+}
+
+hipError_t launch_transition_f32(const TransitionCall& c, hipStream_t stream) {
+  if (c.backward) return launch_transition_f32_t<float, true>(c, stream);
+  return c.dtype == Dtype::BF16 ? launch_transition_f32_t<bf16_t, false>(c, stream)
+                                : launch_transition_f32_t<float, false>(c, stream);
 }
 
 }  // namespace wkv7

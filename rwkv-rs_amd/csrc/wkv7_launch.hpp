@@ -85,6 +85,19 @@ void place_segments(Segments* s, int B, int H, void* workspace);
 // fault words
 hipError_t launch_segment_bounds(const ForwardDesc& d, hipStream_t stream);
 hipError_t launch_segment_bounds(const BackwardDesc& d, hipStream_t stream);
+// the transition pass of a call that runs on the fp32 chunked kernels
+// (wkv7_f32_chunk.hip; the bf16 one's is in wkv7_segment.hip): x, a, b, then k
+// and v (forward) or r and dy (backward)
+struct TransitionCall {
+  const void* in[5];
+  const float* edge;            // the initial state or the final-state gradient, or nullptr
+  Segments seg;
+  int B, T, H;
+  Dtype dtype;
+  bool backward;
+  uint32_t spin_limit;          // > 0
+};
+hipError_t launch_transition_f32(const TransitionCall& c, hipStream_t stream);
 // after a segmented forward: every output of a (batch, head) any of whose
 // segments gave up a wait becomes NaN, and the event is counted once
 hipError_t launch_segment_poison(const ForwardDesc& d, hipStream_t stream);

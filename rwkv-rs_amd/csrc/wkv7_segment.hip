@@ -1,4 +1,6 @@
-// Sequences cut into segments that run side by side (bf16 operands).
+// Sequences cut into segments that run side by side. The transition kernel
+// here is for bf16 operands; the one with fp32 products is in
+// wkv7_f32_chunk.hip, and the combine and poison kernels serve both.
 //
 // One workgroup per (batch, head) walks a whole sequence, so a call with few
 // pairs leaves most of the chip idle for as long as one chain of chunks takes.
@@ -89,7 +91,7 @@ struct SegParams {
   float* trans;           // [B,H,G,64,64]: M of segment g
   int* fault;             // [B,H,G]: segment g's wait gave up
   int T, H, G, cps;       // cps: chunks per segment (the last may have fewer)
-  uint32_t spin_limit;
+  uint32_t spin_limit;    // polls per hand-over wait (> 0)
 };
 
 __device__ __forceinline__ const uint4* seg_piece(const SegParams& p, int64_t tok0, int64_t tstride, int c,
@@ -427,20 +429,28 @@ __global__ __launch_bounds__(64) void wkv7_segment_poison_kernel(const int* faul
 }
 
 template <bool kBwd>
-hipError_t launch_bounds(SegParams& p, int B, int T, int H, const Segments& seg, uint32_t spin_limit,
-                         hipStream_t stream) {
-  p.bound = seg.bound;
-  p.trans = seg.trans;
-  p.fault = seg.fault;
-  p.T = T;
-  p.H = H;
-  p.G = seg.G;
-  p.cps = seg.cps;
-  p.spin_limit = spin_limit ? spin_limit : kSpinLimit;
-  hipLaunchKernelGGL(wkv7_transition_kernel<kBwd>, dim3(H, B, p.G - 1), dim3(kBlock), 0, stream, p);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess || p.G < 3) return e;
-  hipLaunchKernelGGL(wkv7_combine_kernel<kBwd>, dim3(B * H, 4), dim3(256), 0, stream, p.bound, p.trans, p.G);
+hipError_t launch_bounds(const TransitionCall& c, bool f32, hipStream_t stream) {
+  hipError_t e;
+  if (f32) {
+    e = launch_transition_f32(c, stream);
+  } else {
+    SegParams p;
+    for (int i = 0; i < kVecs; ++i) p.in[i] = static_cast<const bf16_t*>(c.in[i]);
+    p.edge = c.edge;
+    p.bound = c.seg.bound;
+    p.trans = c.seg.trans;
+    p.fault = c.seg.fault;
+    p.T = c.T;
+    p.H = c.H;
+    p.G = c.seg.G;
+    p.cps = c.seg.cps;
+    p.spin_limit = c.spin_limit;
+    hipLaunchKernelGGL(wkv7_transition_kernel<kBwd>, dim3(c.H, c.B, p.G - 1), dim3(kBlock), 0, stream, p);
+    e = hipGetLastError();
+  }
+  if (e != hipSuccess || c.seg.G < 3) return e;
+  hipLaunchKernelGGL(wkv7_combine_kernel<kBwd>, dim3(c.B * c.H, 4), dim3(256), 0, stream, c.seg.bound, c.seg.trans,
+                     c.seg.G);
   return hipGetLastError();
 }
 
@@ -459,6 +469,14 @@ constexpr Cost kForwardCost = {22.f, 4.5f, 1.36f, 34.f, 16.f, 0.65f, 3.6f};
 // Backward, 32 pairs: n = 256: 748 and 171; n = 32: 106 and 48; n = 16: 60 and
 // 38. 128 pairs, n = 64: 201 and 150 (2 segments).
 constexpr Cost kBackwardCost = {28.f, 13.f, 2.88f, 37.f, 25.f, 0.65f, 4.38f};
+
+// The fp32 chunked kernels. Forward, 32 pairs: n = 256: 725 in one piece and
+// 222 in 8 segments; n = 32: 101 and 53; n = 16: 54 and 40; 85 pairs, n = 16:
+// 59 and 63 (3 segments).
+constexpr Cost kForwardCost32 = {22.f, 9.f, 2.8f, 34.f, 27.f, 0.5f, 5.7f};
+// Backward, 32 pairs: n = 256: 1922 and 359; n = 16: 130 and 48. 128 pairs, n =
+// 64: 492 and 319 (2 segments).
+constexpr Cost kBackwardCost32 = {28.f, 5.f, 7.6f, 37.f, 25.f, 0.5f, 9.6f};
 
 // The cheapest number of segments, among those whose workgroups (one per pair
 // and segment, each filling a CU's LDS) all run at once: more would queue, and
@@ -485,12 +503,19 @@ Segments plan(int64_t pairs, int n, int q, const Cost& k) {
 }  // namespace
 
 Segments plan_segments(const ForwardDesc& d) {
-  if (d.kc.step_only || !chunk_forward_supported(d)) return Segments{};
-  return plan((int64_t)d.B * d.H, d.T / kL, 1, kForwardCost);
+  const int64_t pairs = (int64_t)d.B * d.H;
+  if (d.kc.step_only) return Segments{};
+  if (chunk_forward_supported(d)) return plan(pairs, d.T / kL, 1, kForwardCost);
+  if (chunk_f32_forward_supported(d)) return plan(pairs, d.T / kL, d.C / kL, kForwardCost32);
+  return Segments{};
 }
 Segments plan_segments(const BackwardDesc& d) {
-  if (d.kc.step_only || !chunk_backward_supported(d)) return Segments{};
-  return plan((int64_t)d.B * d.H, d.T / kL, d.C / kL, kBackwardCost);
+  const int64_t pairs = (int64_t)d.B * d.H;
+  if (d.kc.step_only) return Segments{};
+  if (chunk_backward_supported(d)) return plan(pairs, d.T / kL, d.C / kL, kBackwardCost);
+  if (chunk_f32_backward_supported(d) && chunk_f32_backward_preferred(d))
+    return plan(pairs, d.T / kL, d.C / kL, kBackwardCost32);
+  return Segments{};
 }
 
 int64_t segment_bytes(const Segments& s, int B, int H) {
@@ -505,25 +530,25 @@ void place_segments(Segments* s, int B, int H, void* workspace) {
 }
 
 hipError_t launch_segment_bounds(const ForwardDesc& d, hipStream_t stream) {
-  SegParams p;
-  const void* in[kVecs] = {d.w, d.a, d.b, d.k, d.v};
-  for (int i = 0; i < kVecs; ++i) p.in[i] = static_cast<const bf16_t*>(in[i]);
-  p.edge = d.s0;
-  return launch_bounds<false>(p, d.B, d.T, d.H, d.seg, d.kc.spin_limit, stream);
+  return launch_bounds<false>(TransitionCall{{d.w, d.a, d.b, d.k, d.v}, d.s0, d.seg, d.B, d.T, d.H, d.dtype, false,
+                                             d.kc.spin_limit ? d.kc.spin_limit : kSpinLimit},
+                              !chunk_forward_supported(d), stream);
 }
 hipError_t launch_segment_bounds(const BackwardDesc& d, hipStream_t stream) {
-  SegParams p;
-  const void* in[kVecs] = {d.w, d.a, d.b, d.r, d.dy};
-  for (int i = 0; i < kVecs; ++i) p.in[i] = static_cast<const bf16_t*>(in[i]);
-  p.edge = d.dsT;
-  return launch_bounds<true>(p, d.B, d.T, d.H, d.seg, d.kc.spin_limit, stream);
+  return launch_bounds<true>(TransitionCall{{d.w, d.a, d.b, d.r, d.dy}, d.dsT, d.seg, d.B, d.T, d.H, d.dtype, true,
+                                            d.kc.spin_limit ? d.kc.spin_limit : kSpinLimit},
+                             !chunk_backward_supported(d), stream);
 }
 hipError_t launch_segment_poison(const ForwardDesc& d, hipStream_t stream) {
   unsigned int* faults;
   if (hipError_t e = handover_fault_counter(&faults)) return e;
-  hipLaunchKernelGGL(wkv7_segment_poison_kernel<bf16_t>, dim3(d.H, d.B), dim3(64), 0, stream, d.seg.fault,
-                     d.seg.G, static_cast<bf16_t*>(d.y), d.sa, d.ckpt, d.sT, d.T, d.C, faults);
-  return hipGetLastError();
+  auto go = [&](auto* y) {
+    typedef typename std::remove_pointer<decltype(y)>::type Tio;
+    hipLaunchKernelGGL(wkv7_segment_poison_kernel<Tio>, dim3(d.H, d.B), dim3(64), 0, stream, d.seg.fault, d.seg.G, y,
+                       d.sa, d.ckpt, d.sT, d.T, d.C, faults);
+    return hipGetLastError();
+  };
+  return d.dtype == Dtype::BF16 ? go(static_cast<bf16_t*>(d.y)) : go(static_cast<float*>(d.y));
 }
 
 }  // namespace wkv7
