@@ -4,16 +4,26 @@
 // logits instead of a cast to fp32, a softmax, its backward, a cast back and
 // l2wrap's max / clone / scatter.
 //
-// One block of 256 threads per row. Each thread walks the row in pieces of 8
-// logits (one 16-byte access for bf16 when the vocabulary is a multiple of 8,
-// else element by element), keeping a running maximum m, the sum
-// s of exp(x - m) rescaled whenever m grows, and the first index of m. The
-// 256 partial (m, s, index) triples are combined by wave shuffles and then
-// across the four waves in a fixed order, so a row's result does not depend
-// on scheduling. The backward recomputes exp(x - lse) from the saved
-// log-sum-exp and writes each gradient once.
-#include <cmath>
+// A row is walked in pieces of 8 logits (one 16-byte access for bf16, two for
+// fp32). Rows of a vocabulary that is no multiple of 8 begin anywhere, so the
+// pieces begin at the row's first 16-byte boundary, and the few logits before
+// it and after the last whole piece go one to a thread (RowSpan). Forward: a
+// block per row; each thread keeps a running maximum m, the sum s of exp(x - m)
+// rescaled whenever m grows, and the first index of m. The threads' triples
+// are combined by wave shuffles and then across the waves in a fixed order, so
+// a row's result does not depend on scheduling. The backward recomputes
+// exp(x - lse) from the saved log-sum-exp and writes each gradient once; a
+// row's pieces are independent there, so with few rows several blocks share
+// one.
+//
+// HBM bounds it once the rows fill the chip: 8192 x 65536 bf16, forward 187 us
+// (5.7 TB/s), backward 420 us (5.1). With the logits of a ragged row taken one
+// by one instead of in pieces, 8192 x 65529 took 545 + 1,271 us in bf16 and 898
+// + 2,070 in fp32; in pieces 189 + 450 and 361 + 916 (its rows' edges share
+// cache lines with their neighbours').
+#include <algorithm>
 #include <climits>
+#include <cmath>
 
 #include "lm_loss_launch.hpp"
 
@@ -61,43 +71,31 @@ __device__ __forceinline__ void store_piece(void* base, int64_t i, const Piece& 
   }
 }
 
-// logits j0 .. j0 + 7 of a row: one vector access when every row is a whole
-// number of pieces (VEC), else element by element, -inf past the row's end
-template <bool BF, bool VEC>
-__device__ __forceinline__ Piece load_row(const void* base, int64_t row0, int64_t j0, int64_t V) {
-  if constexpr (VEC) {
-    return load_piece<BF>(base, row0 + j0);
-  } else {
-    Piece p;
-#pragma unroll
-    for (int k = 0; k < kPiece; ++k) {
-      const int64_t j = j0 + k;
-      p.v[k] = j >= V ? -INFINITY
-               : BF   ? __builtin_bit_cast(float, static_cast<uint32_t>(
-                                                    static_cast<const uint16_t*>(base)[row0 + j])
-                                                    << 16)
-                      : static_cast<const float*>(base)[row0 + j];
-    }
-    return p;
-  }
+template <bool BF>
+__device__ __forceinline__ float load_one(const void* base, int64_t i) {
+  if constexpr (BF) return __builtin_bit_cast(float, static_cast<uint32_t>(static_cast<const uint16_t*>(base)[i]) << 16);
+  else return static_cast<const float*>(base)[i];
 }
 
-template <bool BF, bool VEC>
-__device__ __forceinline__ void store_row(void* base, int64_t row0, int64_t j0, int64_t V,
-                                          const Piece& p) {
-  if constexpr (VEC) {
-    store_piece<BF>(base, row0 + j0, p);
-  } else {
-#pragma unroll
-    for (int k = 0; k < kPiece; ++k) {
-      const int64_t j = j0 + k;
-      if (j >= V) break;
-      if constexpr (BF)
-        static_cast<uint16_t*>(base)[row0 + j] = __builtin_bit_cast(uint16_t, static_cast<__bf16>(p.v[k]));
-      else
-        static_cast<float*>(base)[row0 + j] = p.v[k];
-    }
-  }
+template <bool BF>
+__device__ __forceinline__ void store_one(void* base, int64_t i, float v) {
+  if constexpr (BF) static_cast<uint16_t*>(base)[i] = __builtin_bit_cast(uint16_t, static_cast<__bf16>(v));
+  else static_cast<float*>(base)[i] = v;
+}
+
+// Elements [0, head) and [tail, V) of a row are taken one by one, the pieces
+// between them start on a 16-byte boundary. head and V - tail are below kPiece.
+struct RowSpan {
+  int64_t pieces, tail;
+  int head;
+};
+template <bool BF>
+__device__ __forceinline__ RowSpan row_span(const void* base, int64_t row0, int64_t V) {
+  constexpr int kSize = BF ? 2 : 4;
+  const uintptr_t at = reinterpret_cast<uintptr_t>(base) + row0 * kSize;
+  const int head = static_cast<int>(min(static_cast<int64_t>((16 - (at & 15)) & 15) / kSize, V));
+  const int64_t pieces = (V - head) / kPiece;
+  return {pieces, head + pieces * kPiece, head};
 }
 
 // running (max, sum of exp(x - max), first index of max)
@@ -120,14 +118,26 @@ __device__ __forceinline__ Run combine(const Run& a, const Run& b) {
   return r;
 }
 
-template <bool BF, bool VEC>
-__global__ __launch_bounds__(kThreads) void xent_forward_kernel(XentArgs a) {
-  __shared__ Run part[kThreads / 64];
+template <bool BF, int kWidth>
+__global__ __launch_bounds__(kWidth) void xent_forward_kernel(XentArgs a) {
+  __shared__ Run part[kWidth / 64];
   const int64_t row = blockIdx.x;
-  const int64_t V = a.vocab, base = row * V, pieces = (V + kPiece - 1) / kPiece;
+  const int64_t V = a.vocab, base = row * V;
+  const RowSpan span = row_span<BF>(a.logits, base, V);
+  const int tid = threadIdx.x;
   Run run{-INFINITY, 0.f, INT_MAX};
-  for (int64_t q = threadIdx.x; q < pieces; q += kThreads) {
-    const Piece p = load_row<BF, VEC>(a.logits, base, q * kPiece, V);
+  // a logit of -inf adds nothing (and is no maximum), NaN makes the sum NaN
+  auto single = [&](int64_t j) {
+    const float x = load_one<BF>(a.logits, base + j);
+    const Run one{x, x == -INFINITY ? 0.f : __expf(x - x), static_cast<int>(j)};
+    const Run both = combine(run, one);
+    run = {both.m, both.s, x > run.m ? one.idx : run.idx};
+  };
+  // each thread sees its logits by rising index: head, pieces, tail
+  if (tid < span.head) single(tid);
+  for (int64_t q = tid; q < span.pieces; q += kWidth) {
+    const int64_t j0 = span.head + q * kPiece;
+    const Piece p = load_piece<BF>(a.logits, base + j0);
     float cm = p.v[0];
     int ci = 0;
 #pragma unroll
@@ -137,13 +147,15 @@ __global__ __launch_bounds__(kThreads) void xent_forward_kernel(XentArgs a) {
         ci = k;
       }
     const float m = fmaxf(run.m, cm);
+    const float to = m == -INFINITY ? 0.f : m;   // nothing but -inf so far: the exponentials are 0
     float s = scaled(run.s, run.m, m);
 #pragma unroll
-    for (int k = 0; k < kPiece; ++k) s += __expf(p.v[k] - m);
-    if (cm > run.m) run.idx = static_cast<int>(q * kPiece) + ci;
+    for (int k = 0; k < kPiece; ++k) s += __expf(p.v[k] - to);
+    if (cm > run.m) run.idx = static_cast<int>(j0) + ci;
     run.m = m;
     run.s = s;
   }
+  if (span.tail + tid < V) single(span.tail + tid);
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
     Run o;
@@ -152,20 +164,15 @@ __global__ __launch_bounds__(kThreads) void xent_forward_kernel(XentArgs a) {
     o.idx = __shfl_xor(run.idx, off);
     run = combine(run, o);
   }
-  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = run;
+  if ((tid & 63) == 0) part[tid >> 6] = run;
   __syncthreads();
-  if (threadIdx.x == 0) {
+  if (tid == 0) {
     Run r = part[0];
 #pragma unroll
-    for (int w = 1; w < kThreads / 64; ++w) r = combine(r, part[w]);
+    for (int w = 1; w < kWidth / 64; ++w) r = combine(r, part[w]);
     const float lse = r.m + logf(r.s);
     const int64_t t = a.targets[row];
-    float xt = NAN;
-    if (t >= 0 && t < V)
-      xt = a.bf16 ? __builtin_bit_cast(float, static_cast<uint32_t>(
-                                                  static_cast<const uint16_t*>(a.logits)[base + t])
-                                                  << 16)
-                  : static_cast<const float*>(a.logits)[base + t];
+    const float xt = t >= 0 && t < V ? load_one<BF>(a.logits, base + t) : NAN;
     a.row_loss[row] = lse - xt;
     a.row_lse[row] = lse;
     a.row_max[row] = r.m;
@@ -173,30 +180,72 @@ __global__ __launch_bounds__(kThreads) void xent_forward_kernel(XentArgs a) {
   }
 }
 
-template <bool BF, bool VEC>
+// Blocks (row, y) take every gridDim.y-th run of kThreads pieces. kPieces: the
+// rows of the logits and of their gradient begin alike within 16 bytes; else
+// every element is taken by itself.
+template <bool BF, bool kPieces>
 __global__ __launch_bounds__(kThreads) void xent_backward_kernel(XentArgs a) {
   const int64_t row = blockIdx.x;
-  const int64_t V = a.vocab, base = row * V, pieces = (V + kPiece - 1) / kPiece;
+  const int64_t V = a.vocab, base = row * V;
   const float lse = a.lse[row], g = a.row_grad[row];
   const float l2 = a.l2wrap_scale * a.max[row];
   const int64_t t = a.targets[row], am = a.argmax[row];
-  for (int64_t q = threadIdx.x; q < pieces; q += kThreads) {
-    Piece p = load_row<BF, VEC>(a.logits, base, q * kPiece, V);
-    const int64_t j0 = q * kPiece;
+  const int64_t first = static_cast<int64_t>(blockIdx.y) * kThreads + threadIdx.x;
+  const int64_t stride = static_cast<int64_t>(gridDim.y) * kThreads;
+  auto grad = [&](float x, int64_t j) {
+    float d = g * __expf(x - lse);
+    if (j == t) d -= g;
+    if (j == am) d += l2;
+    return d;
+  };
+  auto single = [&](int64_t j) { store_one<BF>(a.logits_grad, base + j, grad(load_one<BF>(a.logits, base + j), j)); };
+  if constexpr (!kPieces) {
+    for (int64_t j = first; j < V; j += stride) single(j);
+  } else {
+    const RowSpan span = row_span<BF>(a.logits, base, V);
+    if (first < span.head) single(first);
+    for (int64_t q = first; q < span.pieces; q += stride) {
+      const int64_t j0 = span.head + q * kPiece;
+      Piece p = load_piece<BF>(a.logits, base + j0);
 #pragma unroll
-    for (int k = 0; k < kPiece; ++k) {
-      float d = g * __expf(p.v[k] - lse);
-      if (j0 + k == t) d -= g;
-      if (j0 + k == am) d += l2;
-      p.v[k] = d;
+      for (int k = 0; k < kPiece; ++k) p.v[k] = grad(p.v[k], j0 + k);
+      store_piece<BF>(a.logits_grad, base + j0, p);
     }
-    store_row<BF, VEC>(a.logits_grad, base, q * kPiece, V, p);
+    if (span.tail + first < V) single(span.tail + first);
   }
 }
 
-template <typename K>
-hipError_t launch(K kernel, const XentArgs& a, hipStream_t s) {
-  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(a.rows)), dim3(kThreads), 0, s, a);
+// A few long rows leave most of the chip idle and each is a chain of loads: four
+// times the threads a row. us, 256 / 1024 threads, bf16: 65536 logits, 64 rows
+// 11.9 / 9.1, 256 rows 12.5 / 9.6, 1024 rows 25.4 / 26.4; 32000 logits, 256 rows
+// 7.6 / 6.9 (fp32 10.0 / 7.4). At 512 rows bf16 gains 0.7-3 and fp32 loses 1.6-2;
+// at 1009 logits, where most of 1024 threads have no piece, 3.8 / 4.6. The line
+// is where every one of them has at least two.
+constexpr int64_t kWideRows = 256;
+constexpr int kWideThreads = 1024;
+constexpr int64_t kWideVocab = 2 * kWideThreads * kPiece;
+
+template <bool BF>
+hipError_t forward(const XentArgs& a, hipStream_t s) {
+  const dim3 grid(static_cast<unsigned>(a.rows));
+  if (a.rows <= kWideRows && a.vocab >= kWideVocab) hipLaunchKernelGGL((xent_forward_kernel<BF, kWideThreads>), grid, dim3(kWideThreads), 0, s, a);
+  else hipLaunchKernelGGL((xent_forward_kernel<BF, kThreads>), grid, dim3(kThreads), 0, s, a);
+  return hipGetLastError();
+}
+
+// Blocks enough to fill the chip (eight of 256 threads a compute unit); a row has
+// at most one for each run of pieces. us without / with, bf16, 65536 logits: 16
+// rows 13.9 / 4.2, 64 rows 14.4 / 4.6, 256 rows 18.5 / 11.3, 1024 rows 46 / 44.
+constexpr int64_t kFillBlocks = 2048;
+
+template <bool BF>
+hipError_t backward(const XentArgs& a, hipStream_t s) {
+  const bool alike = ((reinterpret_cast<uintptr_t>(a.logits) ^ reinterpret_cast<uintptr_t>(a.logits_grad)) & 15) == 0;
+  const int64_t runs = (a.vocab / (alike ? kPiece : 1) + kThreads - 1) / kThreads;
+  const int64_t split = std::max<int64_t>(1, std::min<int64_t>(kFillBlocks / a.rows, runs));
+  const dim3 grid(static_cast<unsigned>(a.rows), static_cast<unsigned>(split));
+  if (alike) hipLaunchKernelGGL((xent_backward_kernel<BF, true>), grid, dim3(kThreads), 0, s, a);
+  else hipLaunchKernelGGL((xent_backward_kernel<BF, false>), grid, dim3(kThreads), 0, s, a);
   return hipGetLastError();
 }
 
@@ -204,20 +253,12 @@ hipError_t launch(K kernel, const XentArgs& a, hipStream_t s) {
 
 hipError_t launch_xent_forward(const XentArgs& a, hipStream_t s) {
   if (a.rows == 0) return hipSuccess;
-  if (a.vocab % kPiece == 0)
-    return a.bf16 ? launch(xent_forward_kernel<true, true>, a, s)
-                  : launch(xent_forward_kernel<false, true>, a, s);
-  return a.bf16 ? launch(xent_forward_kernel<true, false>, a, s)
-                : launch(xent_forward_kernel<false, false>, a, s);
+  return a.bf16 ? forward<true>(a, s) : forward<false>(a, s);
 }
 
 hipError_t launch_xent_backward(const XentArgs& a, hipStream_t s) {
   if (a.rows == 0) return hipSuccess;
-  if (a.vocab % kPiece == 0)
-    return a.bf16 ? launch(xent_backward_kernel<true, true>, a, s)
-                  : launch(xent_backward_kernel<false, true>, a, s);
-  return a.bf16 ? launch(xent_backward_kernel<true, false>, a, s)
-                : launch(xent_backward_kernel<false, false>, a, s);
+  return a.bf16 ? backward<true>(a, s) : backward<false>(a, s);
 }
 
 }  // namespace rwkv_loss

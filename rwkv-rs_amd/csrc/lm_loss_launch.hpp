@@ -8,7 +8,7 @@
 
 namespace rwkv_loss {
 
-constexpr int kThreads = 256;   // one block per row
+constexpr int kThreads = 256;   // of a block, but for the forward of a few long rows
 constexpr int kPiece = 8;       // logits per 16-byte (bf16) or 32-byte (fp32) access
 
 struct XentArgs {

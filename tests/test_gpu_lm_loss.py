@@ -92,3 +92,45 @@ def test_row_statistics_and_out_of_range_target():
     ref = w.double().cpu()[:, None] * (sm - onehot)
     ref[torch.arange(rows), peak] += 1e-4 / rows * logits.double().max(dim=1).values
     assert rel_l2(x.grad.double().cpu().numpy(), ref.numpy()) <= 1e-5
+
+
+@pytest.mark.parametrize("rows,V,dt,offset", [
+    (1, 1, "bf16", 0), (3, 7, "bf16", 0), (9, 8201, "bf16", 0), (513, 2051, "bf16", 0),
+    (5, 4099, "f32", 0), (520, 2057, "f32", 0), (16, 65529, "bf16", 0),
+    (256, 16384, "bf16", 0), (257, 16387, "bf16", 0), (4, 16383, "f32", 0), (6, 16391, "f32", 1),
+    (9, 333, "bf16", 1), (7, 2051, "f32", 3),
+])
+def test_rows_that_begin_anywhere(rows, V, dt, offset):
+    """Heads, pieces and tails of rows at every alignment, on both widths of the
+    forward and with rows shared by blocks in the backward; ``offset`` elements
+    put the logits, not their gradient, off a 16-byte boundary. Some logits are
+    -inf, a masked vocabulary's, over whole pieces. The module's bars."""
+    ll = load_pkg().lm_loss
+    logits, targets, peak = _inputs(rows, V, dt, rows + V)
+    col = torch.arange(V)
+    masked = ((col < 40) | (col >= V - 3)) & (col[None, :] != peak[:, None]) & (
+        col[None, :] != targets[:, None])
+    logits[masked] = float("-inf")
+    dev = torch.device("cuda:0")
+    flat = torch.empty(rows * V + offset, dtype=DT[dt], device=dev)
+    x = flat[offset:].view(rows, V)
+    x.copy_(logits)
+    x = x.detach().requires_grad_(True)
+    announce("cross_entropy_l2wrap", f"rows{rows}_V{V}_{dt}_offset{offset}")
+    got = ll.cross_entropy_l2wrap_rows(x, targets.to(dev), rows)
+    w = torch.linspace(0.5, 2.0, rows, device=dev)
+    got.backward(w)
+    torch.cuda.synchronize()
+    z = logits.double()
+    at = torch.arange(rows)
+    lse = torch.logsumexp(z, dim=1)
+    want = lse - z[at, targets]
+    # loss = lse - x_t in fp32: an error of 1e-5 of the larger term
+    assert bool(((got.double().cpu() - want).abs() <= 1e-5 * (lse.abs() + z[at, targets].abs())).all())
+    ref = torch.softmax(z, dim=1)
+    ref[at, targets] -= 1.0
+    ref *= w.double().cpu()[:, None]
+    ref[at, peak] += 1e-4 / rows * z.max(dim=1).values
+    grad = x.grad.double().cpu()
+    assert rel_l2(grad.numpy(), ref.numpy()) <= (8e-3 if dt == "bf16" else 1e-5)
+    assert bool((grad[masked] == 0).all())
