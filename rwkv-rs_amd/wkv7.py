@@ -26,6 +26,7 @@ outputs are allocated here like its ``empty_device`` (wkv7_common/host.rs:114-13
 from __future__ import annotations
 
 import contextlib
+import functools
 from dataclasses import dataclass
 from typing import List, Optional, Tuple
 
@@ -194,12 +195,23 @@ def _options(kernels: str = "auto", handover_spin_limit: int = 0):
     return _native.Wkv7Options(codes[kernels], int(handover_spin_limit))
 
 
+@functools.lru_cache(maxsize=256)
+def _workspace_bytes(query: str, *shape) -> int:
+    """The library's answer for a call without options, a function of the sizes
+    alone. Asked anew on each call it added 1 us to a forward or a backward: B=2,
+    T=96, H=4, both, 44.3-45.1 us; so 43.0-43.7, without a workspace 42.5-43.0."""
+    return getattr(_native.lib(), query)(*shape, None)
+
+
 def _workspace(query: str, B, T, H, N, chunk_len, dtype, options, dev):
     """The workspace a call is cut into segments with (include/wkv7_segments.h),
     as (tensor or None, bytes). Allocated per call on the current stream: the
     caching allocator hands the same block out again."""
-    nbytes = getattr(_native.lib(), query)(B, T, H, N, chunk_len, dtype,
-                                           _native.options_ref(options))
+    if options is None:
+        nbytes = _workspace_bytes(query, B, T, H, N, chunk_len, dtype)
+    else:
+        nbytes = getattr(_native.lib(), query)(B, T, H, N, chunk_len, dtype,
+                                               _native.options_ref(options))
     if nbytes <= 0:
         return None, 0
     return torch.empty(nbytes, dtype=torch.uint8, device=dev), nbytes
