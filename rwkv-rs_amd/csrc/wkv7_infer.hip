@@ -258,7 +258,7 @@ __global__ __launch_bounds__(kRowsBlock) void wkv7_infer_rows_kernel(InferParams
       }
       lds_barrier();
     }
-    outputs(ntiles - 1);
+    if (ntiles > 0) outputs(ntiles - 1);
     return;
   }
 
@@ -725,7 +725,7 @@ hipError_t launch_infer_t(const InferDesc& d, hipStream_t stream) {
 }  // namespace
 
 hipError_t launch_infer(const InferDesc& d, hipStream_t stream) {
-  if (d.Ba == 0 || d.H == 0) return hipSuccess;
+  if (d.Ba == 0 || d.H == 0 || d.T == 0) return hipSuccess;   // no step: no output, the states stay
   if (infer_prompt_preferred(d)) return launch_infer_prompt(d, stream);
   if (d.state_dtype == Dtype::BF16) return launch_infer_bf16(d, stream);
   return d.dtype == Dtype::BF16 ? launch_infer_t<bf16_t>(d, stream) : launch_infer_t<float>(d, stream);

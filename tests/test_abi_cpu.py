@@ -165,6 +165,20 @@ def test_infer_validation(native):
     assert inf(Ba=0, sdtype=1) == 0
 
 
+def test_infer_without_tokens_launches_nothing(native):
+    # empty tensors have null pointers; a launch would be WKV7_ERR_HIP, where
+    # there is no GPU. 8 and 512 (row, head) pairs: both sides of the line
+    # between the kernels for several steps
+    torch = pytest.importorskip("torch")
+    if torch.cuda.is_available():
+        pytest.skip("a launch fails only where there is no GPU")
+    lib = native.lib()
+    for rows in (2, 128):
+        for dtype, sdtype in ((0, 0), (1, 0), (1, 1)):
+            assert lib.wkv7_infer_forward(*([None] * 6), FAKE * 10, FAKE * 1000, None, FAKE * 20, rows, 0,
+                                          4, 64, rows, dtype, sdtype, sdtype, None, None) == 0
+
+
 def test_python_mirror_checks_chunk_len_before_the_gpu():
     pytest.importorskip("torch")
     wk = load_pkg().wkv7

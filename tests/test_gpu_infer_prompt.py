@@ -98,3 +98,18 @@ def test_fp32_state_prompts_equal_a_larger_call(dtype, rows, T, H, mask):
     assert torch.equal(small[used], big[used])
     rest = ids[rows:].long()
     assert torch.equal(small[rest], state[rest])
+
+
+@pytest.mark.parametrize("rows", [2, 130])                  # below and above 256 pairs
+@pytest.mark.parametrize("dtype,state_dtype", [
+    (torch.float32, torch.float32), (torch.bfloat16, torch.float32), (torch.bfloat16, torch.bfloat16)])
+def test_a_call_without_tokens_leaves_the_states(rows, dtype, state_dtype):
+    announce("prompt of no tokens", rows, str(dtype), str(state_dtype))
+    wk = load_pkg().wkv7
+    ops = [torch.empty(rows, 0, 2, 64, dtype=dtype, device="cuda") for _ in range(6)]
+    st = torch.randn(rows, 2, 64, 64, device="cuda").to(state_dtype)
+    before = st.clone()
+    out = wk.wkv7_infer_forward(*ops, torch.arange(rows, dtype=torch.int32, device="cuda"), st, None,
+                                torch.zeros(rows, dtype=torch.int32, device="cuda"))
+    torch.cuda.synchronize()
+    assert out.output.shape == (rows, 0, 2, 64) and torch.equal(st, before)
