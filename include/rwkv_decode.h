@@ -59,8 +59,9 @@ int64_t rwkv_decode_workspace_bytes(int64_t rows, int64_t num_heads);
  * works on slot batch_ids[b] of state ([full_batch, num_heads, 64, 64] in
  * state_dtype, updated in place) and of the token shifts ([full_batch, C]
  * fp32: read from shift_*_in, written whole to shift_*_out, another buffer;
- * other slots are copied). batch_ids must be distinct; a row whose id is out
- * of range works on zeros and touches no slot. use_dither and elapsed_t as in
+ * other slots are copied). batch_ids must be distinct, so more rows than slots
+ * are refused (WKV7_ERR_SHAPE); a row whose id is out of range works on zeros
+ * and touches no slot. use_dither and elapsed_t as in
  * wkv7_infer_forward. params->residual_a == NULL marks the first cell. */
 int rwkv_decode_cell(const rwkv_decode_cell_params *params, float *x,
                      const int32_t *batch_ids, void *state,

@@ -48,7 +48,8 @@ int rwkv_decode_cell(const rwkv_decode_cell_params* params, float* x, const int3
                      int64_t full_batch, int state_dtype, int use_dither, void* workspace,
                      int64_t workspace_bytes, void* stream) {
   if (state_dtype != WKV7_DTYPE_F32 && state_dtype != WKV7_DTYPE_BF16) return WKV7_ERR_DTYPE;
-  if (!supported(rows, num_heads) || full_batch < 0 || full_batch > INT32_MAX - RWKV_DECODE_MAX_ROWS)
+  // distinct ids need as many slots, as in wkv7_infer_forward
+  if (!supported(rows, num_heads) || full_batch < rows || full_batch > INT32_MAX - RWKV_DECODE_MAX_ROWS)
     return WKV7_ERR_SHAPE;
   if (use_dither != 0 && use_dither != 1) return WKV7_ERR_FLAGS;
   if (use_dither && state_dtype == WKV7_DTYPE_F32) return WKV7_ERR_FLAGS;
@@ -66,7 +67,6 @@ int rwkv_decode_cell(const rwkv_decode_cell_params* params, float* x, const int3
   if (p.residual_a)
     if (int rc = check_pointers({p.residual_a, p.residual_b, p.residual_bias})) return rc;
   if (rows == 0) return WKV7_OK;
-  if (full_batch == 0) return WKV7_ERR_SHAPE;
   if (int rc = check_pointers({x, state, shift_time_in, shift_time_out, shift_channel_in, shift_channel_out, workspace}))
     return rc;
   if (!batch_ids || (use_dither && !elapsed_t)) return WKV7_ERR_NULL_POINTER;

@@ -116,3 +116,16 @@ def test_an_id_out_of_range_touches_no_slot():
     for x, y in zip(st.state + st.shift_time + st.shift_channel,
                     ref.state + ref.shift_time + ref.shift_channel):
         assert torch.equal(x[[0, 1, 3]], y[[0, 1, 3]]) and not torch.equal(x[2], y[2])
+
+
+def test_more_rows_than_slots_are_refused():
+    announce("decode step, more rows than slots")
+    model = _model()
+    st, ref = _state(model, 2, torch.bfloat16, 2), _state(model, 2, torch.bfloat16, 2)
+    toks = torch.arange(3, device=DEV).reshape(3, 1)
+    with pytest.raises(load_pkg()._native.Wkv7Error, match="WKV7_ERR_SHAPE"):
+        _infer(model, toks, torch.tensor([0, 1, 1], device=DEV), st)
+    torch.cuda.synchronize()
+    for x, y in zip(st.state + st.shift_time + st.shift_channel,
+                    ref.state + ref.shift_time + ref.shift_channel):
+        assert torch.equal(x, y)
