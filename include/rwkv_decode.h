@@ -61,7 +61,8 @@ int64_t rwkv_decode_workspace_bytes(int64_t rows, int64_t num_heads);
  * fp32: read from shift_*_in, written whole to shift_*_out, another buffer;
  * other slots are copied). batch_ids must be distinct, so more rows than slots
  * are refused (WKV7_ERR_SHAPE); a row whose id is out of range works on zeros
- * and touches no slot. use_dither and elapsed_t as in
+ * and touches no slot. What a call writes may overlap neither each other nor
+ * what it reads (WKV7_ERR_OVERLAP). use_dither and elapsed_t as in
  * wkv7_infer_forward. params->residual_a == NULL marks the first cell. */
 int rwkv_decode_cell(const rwkv_decode_cell_params *params, float *x,
                      const int32_t *batch_ids, void *state,

@@ -8,7 +8,7 @@ import pytest
 from conftest import load_pkg
 
 F32, BF16 = 0, 1
-NULL, SHAPE = 1, 2
+NULL, SHAPE, ALIGNMENT, OVERLAP = 1, 2, 6, 7
 HIP = 9            # past the checks: the launch, where there is no GPU
 GIB = 1 << 30      # spacing of addresses that are never dereferenced
 
@@ -56,6 +56,42 @@ def test_a_cell_refuses_what_the_recurrence_refuses(native, first):
     assert _cell(native, p, rows=5) == SHAPE                    # more rows than slots
     assert _cell(native, p, rows=1, slots=0) == SHAPE
     assert _cell(native, p, rows=0, slots=0) == 0
+    assert _cell(native, p, ids=2 * GIB + 2) == ALIGNMENT
+    assert _cell(native, p, et=8 * GIB + 1) == ALIGNMENT
     assert _cell(native, p, et=None) == NULL
     assert _cell(native, p, dtype=F32, dither=0, et=None) == HIP
     assert _cell(native, p, nbytes=16) == SHAPE
+
+
+@pytest.mark.parametrize("first", [True, False])
+def test_a_cell_refuses_overlap(native, first):
+    p = _params(native, first)
+    row, shift, state = 128 * 4, 4 * 128 * 4, 4 * 2 * 64 * 64 * 2
+    ends = dict(x=3 * row, state=state, to=shift, co=shift,
+                ws=native.lib().rwkv_decode_workspace_bytes(3, 2))
+    ins = dict(ids=2 * GIB, ti=4 * GIB, ci=6 * GIB, et=8 * GIB)
+    for name, size in ends.items():
+        for other, at in ins.items():           # over the input's first bytes, and just before it
+            assert _cell(native, p, **{name: at}) == OVERLAP, (name, other)
+            assert _cell(native, p, **{name: at - size + 16}) == OVERLAP, (name, other)
+            assert _cell(native, p, **{name: at - size}) == HIP, (name, other)
+        at = p.channel_value
+        assert _cell(native, p, **{name: at + 4 * 128 * 128 * 4 - 16}) == OVERLAP, name
+        assert _cell(native, p, **{name: at + 4 * 128 * 128 * 4}) == HIP, name
+        if not first:
+            assert _cell(native, p, **{name: p.residual_b}) == OVERLAP, name
+    assert _cell(native, p, x=3 * GIB + state - 16) == OVERLAP  # two that are written
+    assert _cell(native, p, to=7 * GIB) == OVERLAP
+    assert _cell(native, p, ws=5 * GIB) == OVERLAP
+
+
+def test_a_head_refuses_overlap(native):
+    lib = native.lib()
+    need = lib.rwkv_decode_workspace_bytes(3, 2)
+
+    def head(x=GIB, w=2 * GIB, b=3 * GIB, un=4 * GIB, logits=5 * GIB, ws=6 * GIB):
+        return lib.rwkv_decode_head(x, w, b, 1e-5, un, 3, 2, 50, logits, ws, need, None)
+    assert head() == HIP
+    assert head(logits=GIB + 3 * 128 * 4 - 16) == OVERLAP
+    assert head(logits=2 * GIB) == OVERLAP and head(ws=4 * GIB + 50 * 128 * 4 - 16) == OVERLAP
+    assert head(ws=5 * GIB) == OVERLAP and head(ws=5 * GIB + 304) == HIP   # 3 x 50 logits end at 300
