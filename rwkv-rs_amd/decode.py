@@ -182,8 +182,10 @@ def step(model, contexts, batch_ids, infer_state, context_mask,
     ids = batch_ids.to(device=dev, dtype=torch.int32).contiguous()
     elapsed = infer_state.elapsed_t.to(device=dev, dtype=torch.int32).contiguous()
     x = model.layer_norm_for_first_cell(model.embed(contexts))
-    if x.dtype != torch.float32 or not x.is_contiguous() or x.shape != (rows, 1, C):
+    if x.dtype != torch.float32 or x.shape != (rows, 1, C):
         return None
+    # the cells add to it in place, and a hook or the norm itself may hold x
+    x = x.clone(memory_format=torch.contiguous_format)
     lib = _native.lib()
     nbytes = lib.rwkv_decode_workspace_bytes(rows, H)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)

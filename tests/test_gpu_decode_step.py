@@ -129,3 +129,26 @@ def test_more_rows_than_slots_are_refused():
     for x, y in zip(st.state + st.shift_time + st.shift_channel,
                     ref.state + ref.shift_time + ref.shift_channel):
         assert torch.equal(x, y)
+
+
+def test_the_first_norms_output_is_not_written():
+    # what a hook on it keeps (activation capture), or the norm itself
+    announce("decode step, the first norm's output kept by others")
+    model = _model()
+    ids, toks = torch.arange(3, device=DEV), torch.arange(3, device=DEV).reshape(3, 1)
+    plain = _infer(model, toks, ids, _state(model, 4, torch.bfloat16, 1))
+    kept = []
+    hook = model.layer_norm_for_first_cell.register_forward_hook(lambda m, i, out: kept.append(out))
+    hooked = _infer(model, toks, ids, _state(model, 4, torch.bfloat16, 1))
+    hook.remove()
+    want = model.layer_norm_for_first_cell(model.embed(toks))
+    assert len(kept) == 1 and torch.equal(kept[0], want) and torch.equal(hooked, plain)
+
+    class Kept(torch.nn.Module):
+        def forward(self, x):
+            return want
+    model.layer_norm_for_first_cell = Kept()
+    before = want.clone()
+    for _ in range(2):
+        assert torch.equal(_infer(model, toks, ids, _state(model, 4, torch.bfloat16, 1)), plain)
+    assert torch.equal(want, before)
