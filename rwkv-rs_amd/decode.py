@@ -183,7 +183,8 @@ def step(model, contexts, batch_ids, infer_state, context_mask,
     elapsed = infer_state.elapsed_t.to(device=dev, dtype=torch.int32).contiguous()
     x = model.layer_norm_for_first_cell(model.embed(contexts))
     if x.dtype != torch.float32 or x.shape != (rows, 1, C):
-        return None
+        # the embedding and the norm have run, and run once a step
+        return (model._infer_cells(x, T, batch_ids, infer_state, context_mask, unembed_mode),)
     # the cells add to it in place, and a hook or the norm itself may hold x
     x = x.clone(memory_format=torch.contiguous_format)
     lib = _native.lib()

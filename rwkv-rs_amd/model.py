@@ -627,10 +627,13 @@ class AutoRegressiveModel(nn.Module):
         fused = _decode.step(self, contexts, batch_ids, infer_state, context_mask, unembed_mode)
         if fused is not None:
             return fused[0]
-        kernel = _wkv7.KernelInfer
         x = self.layer_norm_for_first_cell(self.embed(contexts))
-        x, st, state, sc = self.cells(x, batch_ids, kernel, infer_state.elapsed_t, context_mask,
-                                      infer_state.shift_time, infer_state.state,
+        return self._infer_cells(x, T, batch_ids, infer_state, context_mask, unembed_mode)
+
+    def _infer_cells(self, x, T, batch_ids, infer_state, context_mask, unembed_mode):
+        """``infer`` of T steps from the first cell on."""
+        x, st, state, sc = self.cells(x, batch_ids, _wkv7.KernelInfer, infer_state.elapsed_t,
+                                      context_mask, infer_state.shift_time, infer_state.state,
                                       infer_state.shift_channel)
         infer_state.shift_time[:] = st
         infer_state.state[:] = state

@@ -152,3 +152,27 @@ def test_the_first_norms_output_is_not_written():
     for _ in range(2):
         assert torch.equal(_infer(model, toks, ids, _state(model, 4, torch.bfloat16, 1)), plain)
     assert torch.equal(want, before)
+
+
+def test_the_embedding_and_the_first_norm_run_once(monkeypatch):
+    # a first norm whose result the kernels do not take: the modules go on from it
+    announce("decode step, a first norm in bf16")
+    decode = load_pkg().decode
+    model = _model()
+    ids, toks = torch.arange(3, device=DEV), torch.arange(3, device=DEV).reshape(3, 1)
+    calls = []
+
+    class Norm(torch.nn.Module):
+        def forward(self, x):
+            calls.append("norm")
+            return x.bfloat16()
+    model.layer_norm_for_first_cell = Norm()
+    model.embed.register_forward_hook(lambda *x: calls.append("embed"))
+    a, b = _state(model, 4, torch.bfloat16, 1), _state(model, 4, torch.bfloat16, 1)
+    got = _infer(model, toks, ids, a)
+    assert calls == ["embed", "norm"]
+    assert _infer(model, toks, ids, _state(model, 4, torch.bfloat16, 1), "skip") is None
+    monkeypatch.setattr(decode, "step", lambda *x: None)
+    assert torch.equal(got, _infer(model, toks, ids, b))
+    for x, y in zip(a.state + a.shift_time + a.shift_channel, b.state + b.shift_time + b.shift_channel):
+        assert x.dtype == y.dtype and torch.equal(x, y)
