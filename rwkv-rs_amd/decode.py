@@ -6,9 +6,10 @@ modules' forwards one after another: nine launches a cell issued by one native
 call, against about sixty from Python. Everything is read from the modules on
 every call, and nothing is kept between calls.
 
-The modules are passed by, so anything attached to one of them (a hook, a
-replaced or subclassed module, a forward set on the instance) sends the whole
-step back to the modules.
+The embedding and the first layer norm run as the modules they are. The cells
+and the head are passed by, so anything attached to one of their modules (a
+hook, a replaced or subclassed module, a parameter that is no longer one, a
+forward set on the instance) sends the whole step back to the modules.
 """
 
 from __future__ import annotations
@@ -26,10 +27,12 @@ MAX_DIM = 8192       # RWKV_DECODE_MAX_DIM
 
 
 def _plain(module, cls) -> bool:
-    """Exactly ``cls``, calling nothing but its own forward."""
+    """Exactly ``cls`` (a missing module, None, is not), calling nothing but
+    its own forward."""
+    if type(module) is not cls:
+        return False
     d = module.__dict__
-    return (type(module) is cls and not d["_forward_hooks"] and not d["_forward_pre_hooks"]
-            and "forward" not in d)
+    return not d["_forward_hooks"] and not d["_forward_pre_hooks"] and "forward" not in d
 
 
 class _Unsupported(Exception):
@@ -53,15 +56,17 @@ class _Reader:
         return p
 
     def param(self, module, name, shape) -> int:
-        return self.tensor(module._parameters[name], shape)
+        """A parameter; one replaced by another kind of attribute is not taken."""
+        return self.tensor(module._parameters.get(name), shape)
 
     def linear(self, module, d_in, d_out) -> int:
-        if not _plain(module, nn.Linear) or module._parameters["bias"] is not None:
+        if not _plain(module, nn.Linear) or module._parameters.get("bias", self) is not None:
             raise _Unsupported
         return self.param(module, "weight", (d_out, d_in))
 
     def norm(self, module, dim):
-        if not _plain(module, nn.LayerNorm) or module.normalized_shape != (dim,):
+        if (not _plain(module, nn.LayerNorm) or module.normalized_shape != (dim,)
+                or not 0.0 <= module.eps < float("inf")):
             raise _Unsupported
         return (self.param(module, "weight", (dim,)), self.param(module, "bias", (dim,)),
                 float(module.eps))
@@ -69,11 +74,13 @@ class _Reader:
 
 def _cell_params(m, cell, rd: _Reader, C: int, H: int):
     """The rwkv_decode_cell_params of one CausalCell."""
-    sub = cell._modules
-    tm, cm = sub["time_mixer"], sub["channel_mixer"]
-    if not (_plain(cell, m.CausalCell) and _plain(tm, m.TimeMixer) and _plain(cm, m.ChannelMixer)):
+    if not _plain(cell, m.CausalCell):
         raise _Unsupported
-    wp, gr = tm._modules["weight_prepare"], tm._modules["gated_readout"]
+    sub = cell._modules
+    tm, cm = sub.get("time_mixer"), sub.get("channel_mixer")
+    if not (_plain(tm, m.TimeMixer) and _plain(cm, m.ChannelMixer)):
+        raise _Unsupported
+    wp, gr = tm._modules.get("weight_prepare"), tm._modules.get("gated_readout")
     if not (_plain(wp, m.WeightPrepare) and _plain(gr, m.GatedReadout)):
         raise _Unsupported
     if (not tm.neighbor_ops == wp.neighbor_ops == gr.neighbor_ops == cm.neighbor_ops == "hip"
@@ -82,36 +89,40 @@ def _cell_params(m, cell, rd: _Reader, C: int, H: int):
         raise _Unsupported
     p = _native.DecodeCellParams()
     p.norm_time_weight, p.norm_time_bias, p.norm_time_eps = rd.norm(
-        sub["pre_layer_norm_for_time_mix"], C)
+        sub.get("pre_layer_norm_for_time_mix"), C)
     p.norm_channel_weight, p.norm_channel_bias, p.norm_channel_eps = rd.norm(
-        sub["pre_layer_norm_for_channel_mix"], C)
+        sub.get("pre_layer_norm_for_channel_mix"), C)
     row = (1, 1, C)
     for i, name in enumerate(("receptance", "weight_decay", "key", "value", "learning_rate")):
         p.mix[i] = rd.param(wp, "param_" + name, row)
     p.mix[5] = rd.param(gr, "param_gate", row)
     wsub, gsub = wp._modules, gr._modules
-    p.receptance = rd.linear(wsub["projection_receptance"], C, C)
-    p.key = rd.linear(wsub["projection_key"], C, C)
-    p.value = rd.linear(wsub["projection_value"], C, C)
-    p.output = rd.linear(gsub["projection_output"], C, C)
+    p.receptance = rd.linear(wsub.get("projection_receptance"), C, C)
+    p.key = rd.linear(wsub.get("projection_key"), C, C)
+    p.value = rd.linear(wsub.get("projection_value"), C, C)
+    p.output = rd.linear(gsub.get("projection_output"), C, C)
 
     def lora(module, activation, bias):
-        if not _plain(module, m.LoRA) or module.activation != activation:
+        # the modules call the LoRA's product, or its forward, which does
+        if (not _plain(module, m.LoRA) or module.activation != activation
+                or "product" in module.__dict__):
             raise _Unsupported
-        a = module._parameters["w_a"]
-        rank = a.shape[-1]
+        a = module._parameters.get("w_a")
+        if a is None or a.dim() != 2:
+            raise _Unsupported
+        rank = a.shape[1]
         out = [rd.tensor(a, (C, rank)), rd.param(module, "w_b", (rank, C)), rank]
         if bias:
             out.append(rd.param(module, "bias", row))
-        elif module._parameters.get("bias") is not None:
+        elif module.__dict__.get("bias", rd) is not None:
             raise _Unsupported
         return out
     p.decay_a, p.decay_b, p.decay_rank, p.decay_bias = lora(
-        wsub["param_weight_decay_lora"], "tanh", True)
+        wsub.get("param_weight_decay_lora"), "tanh", True)
     p.rate_a, p.rate_b, p.rate_rank, p.rate_bias = lora(
-        wsub["param_learning_rate_lora"], "none", True)
-    p.gate_a, p.gate_b, p.gate_rank = lora(gsub["param_output_gate_lora"], "sigmoid", False)
-    residual = wsub["param_value_residual_lora"] if wp.cell_id != 0 else None
+        wsub.get("param_learning_rate_lora"), "none", True)
+    p.gate_a, p.gate_b, p.gate_rank = lora(gsub.get("param_output_gate_lora"), "sigmoid", False)
+    residual = wsub.get("param_value_residual_lora") if wp.cell_id != 0 else None
     if residual is not None:
         p.residual_a, p.residual_b, p.residual_rank, p.residual_bias = lora(residual, "none", True)
     elif wp.cell_id != 0:
@@ -119,15 +130,15 @@ def _cell_params(m, cell, rd: _Reader, C: int, H: int):
     p.key_removal = rd.param(wp, "param_key_removal", row)
     p.key_replacement = rd.param(wp, "param_key_replacement", row)
     p.bonus = rd.param(gr, "param_receptance_key_bonus", (H, 64))
-    gn = gsub["group_norm"]
+    gn = gsub.get("group_norm")
     if type(gn) is not nn.GroupNorm:
         raise _Unsupported
     p.group_norm_weight = rd.param(gn, "weight", (C,))
     p.group_norm_bias = rd.param(gn, "bias", (C,))
     p.group_norm_eps = m.GROUP_NORM_EPS
     p.channel_mix = rd.param(cm, "token_shift_diff_scale", row)
-    p.channel_key = rd.linear(cm._modules["key"], C, 4 * C)
-    p.channel_value = rd.linear(cm._modules["value"], 4 * C, C)
+    p.channel_key = rd.linear(cm._modules.get("key"), C, 4 * C)
+    p.channel_value = rd.linear(cm._modules.get("value"), 4 * C, C)
     for rank in (p.decay_rank, p.rate_rank, p.gate_rank, p.residual_rank or 32):
         if rank % 32 or not 0 < rank <= C:
             raise _Unsupported
@@ -144,21 +155,22 @@ def step(model, contexts, batch_ids, infer_state, context_mask,
     GPU, and a model made of the framework's own modules."""
     from . import model as m
     rows, T = contexts.shape
-    dev = model.embed.weight.device
+    if not infer_state.state or infer_state.elapsed_t is None:
+        return None
+    dev = infer_state.state[0].device
     if (T != 1 or not 0 < rows <= MAX_ROWS or context_mask is not None or dev.type != "cuda"
             or model.neighbor_ops != "hip" or not torch.is_autocast_enabled("cuda")
             or torch.get_autocast_dtype("cuda") is not torch.bfloat16
             or nn.modules.module._global_forward_hooks
             or nn.modules.module._global_forward_pre_hooks):
         return None
-    stack = model._modules["cells"]
-    if not _plain(stack, m.MultiCausalCells):
+    stack = model._modules.get("cells")
+    if not _plain(stack, m.MultiCausalCells) or type(stack._modules.get("cells")) is not nn.ModuleList:
         return None
     cells = list(stack._modules["cells"])
-    slots = infer_state.elapsed_t.shape[0]
-    C = model.embed.weight.shape[1]
-    H = C // 64
-    if (not cells or C % 64 or C > MAX_DIM or batch_ids.shape != (rows,)
+    slots, H = infer_state.state[0].shape[:2]
+    C = 64 * H
+    if (not 0 < C <= MAX_DIM or batch_ids.shape != (rows,) or infer_state.elapsed_t.shape != (slots,)
             or not len(infer_state.state) == len(infer_state.shift_time)
             == len(infer_state.shift_channel) == len(cells)):
         return None
@@ -175,8 +187,8 @@ def step(model, contexts, batch_ids, infer_state, context_mask,
             return None   # the first cell is the one without a value residual
         head = None
         if unembed_mode != "skip":
-            head = (rd.norm(model._modules["layer_norm_for_unembed"], C),
-                    rd.linear(model._modules["unembed"], C, model.vocab_size))
+            head = (rd.norm(model._modules.get("layer_norm_for_unembed"), C),
+                    rd.linear(model._modules.get("unembed"), C, model.vocab_size))
     except _Unsupported:
         return None
     ids = batch_ids.to(device=dev, dtype=torch.int32).contiguous()

@@ -176,3 +176,80 @@ def test_the_embedding_and_the_first_norm_run_once(monkeypatch):
     assert torch.equal(got, _infer(model, toks, ids, b))
     for x, y in zip(a.state + a.shift_time + a.shift_channel, b.state + b.shift_time + b.shift_channel):
         assert x.dtype == y.dtype and torch.equal(x, y)
+
+
+class _Wrap(torch.nn.Module):
+    def __init__(self, inner):
+        super().__init__()
+        self.inner = inner
+
+    def forward(self, *args, **kwargs):
+        return self.inner(*args, **kwargs)
+
+
+class _Table(torch.nn.Module):
+    def __init__(self, table):
+        super().__init__()
+        self.register_buffer("table", table)
+
+    def forward(self, ids):
+        return self.table[ids]
+
+
+def _as_attribute(module, name):
+    value = getattr(module, name).detach()
+    delattr(module, name)
+    setattr(module, name, value)
+
+
+def _wrap(module, name):
+    setattr(module, name, _Wrap(getattr(module, name)))
+
+
+def _list_of_cells(model):
+    cells = list(model.cells.cells)
+    del model.cells.cells
+    model.cells.cells = cells
+
+
+@pytest.mark.parametrize("change", [
+    lambda m: m.cells.cells.__setitem__(1, _Wrap(m.cells.cells[1])),
+    lambda m: _wrap(m.cells.cells[0], "time_mixer"),
+    lambda m: _wrap(m.cells.cells[0].time_mixer, "weight_prepare"),
+    lambda m: _wrap(m, "cells"),
+    _list_of_cells,
+    lambda m: _as_attribute(m.cells.cells[1].channel_mixer.value, "weight"),
+    lambda m: _as_attribute(m.cells.cells[1].pre_layer_norm_for_time_mix, "bias"),
+    lambda m: _as_attribute(m.cells.cells[0].time_mixer.weight_prepare, "param_key"),
+    lambda m: _as_attribute(m.cells.cells[0].time_mixer.weight_prepare.param_weight_decay_lora, "w_a"),
+    lambda m: _as_attribute(m.cells.cells[0].time_mixer.weight_prepare.param_weight_decay_lora, "bias"),
+    lambda m: _as_attribute(m.layer_norm_for_unembed, "weight"),
+    lambda m: setattr(m.cells.cells[0].time_mixer.weight_prepare.param_weight_decay_lora, "product",
+                      lambda x: x.float() * 0.0),
+    lambda m: setattr(m, "embed", _Table(m.embed.weight.detach())),
+], ids=["cell", "time_mixer", "weight_prepare", "cells", "list", "linear", "norm", "scale", "lora", "lora_bias",
+        "head_norm", "product", "embed"])
+def test_a_changed_model_still_runs(monkeypatch, request, change):
+    announce("decode step, a changed model", request.node.name)
+    decode = load_pkg().decode
+    model = _model()
+    ids, toks = torch.arange(3, device=DEV), torch.arange(3, device=DEV).reshape(3, 1)
+    plain = _infer(model, toks, ids, _state(model, 4, torch.bfloat16, 1))
+    st = [_state(model, 4, torch.bfloat16, 1) for _ in range(2)]
+    change(model)
+    got = _infer(model, toks, ids, st[0])
+    if "embed" in request.node.callspec.id:      # the kernels do not look at it
+        assert torch.equal(got, plain)
+        return
+    monkeypatch.setattr(decode, "step", lambda *x: None)
+    assert torch.equal(got, _infer(model, toks, ids, st[1]))
+    assert all(torch.equal(x, y) for x, y in zip(st[0].state + st[0].shift_time, st[1].state + st[1].shift_time))
+
+
+def test_a_state_without_elapsed_t_is_refused_as_by_the_modules():
+    announce("decode step, no elapsed_t")
+    model = _model()
+    st = _state(model, 4, torch.float32, 1)
+    st.elapsed_t = None
+    with pytest.raises(ValueError, match="elapsed_t required"):
+        _infer(model, torch.zeros(2, 1, dtype=torch.long, device=DEV), torch.arange(2, device=DEV), st)
