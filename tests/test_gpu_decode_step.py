@@ -225,7 +225,7 @@ def _list_of_cells(model):
     lambda m: _as_attribute(m.cells.cells[0].time_mixer.weight_prepare.param_weight_decay_lora, "bias"),
     lambda m: _as_attribute(m.layer_norm_for_unembed, "weight"),
     lambda m: setattr(m.cells.cells[0].time_mixer.weight_prepare.param_weight_decay_lora, "product",
-                      lambda x: x.float() * 0.0),
+                      lambda x: x * 0.0),
     lambda m: setattr(m, "embed", _Table(m.embed.weight.detach())),
 ], ids=["cell", "time_mixer", "weight_prepare", "cells", "list", "linear", "norm", "scale", "lora", "lora_bias",
         "head_norm", "product", "embed"])
