@@ -183,10 +183,18 @@ __global__ __launch_bounds__(kThreads) void wkv7_infer_kernel(InferParams<Tin> p
 // workgroups of eight such waves; four more waves of each stage the next tile's
 // operands (the decays' exponentials among them) and write the last one's
 // outputs beside them. Sums run in the same order, so the results are the same
-// bit for bit. T = 256, us, the kernel above and this one: 12 pairs 74 / 46, 64
-// pairs 76 / 48, 128 pairs 76 / 50, 256 pairs 82 / 78, 512 pairs 116 / 139. Four
-// workgroups of 16 rows took the same time up to 128 pairs; without the staging
-// waves, whose work the eight then share, 54 us at 36 pairs.
+// bit for bit. us, the kernel above and this one, bf16 operands (fp32 ones are
+// alike up to T = 64):
+//          T = 1      T = 2      T = 4      T = 16     T = 64       T = 256
+//   12     4.0 / 4.1  4.2 / 4.2  4.5 / 4.4  7.4 / 6.1  21.0 / 14.4  74.5 / 46.8
+//   128    4.1 / 4.3  4.4 / 4.5  4.8 / 4.8  7.9 / 6.8  21.9 / 16.0  75.7 / 50.3
+//   144    4.2 / 4.7  4.5 / 4.8  4.9 / 5.2  7.8 / 8.4  21.8 / 22.2  80.8 / 75.2
+//   256    4.4 / 5.0  4.7 / 5.1  5.2 / 5.7  8.4 / 9.1  23.1 / 23.5  86.1 / 85.7
+// (pairs to the left; fp32 operands at T = 256: 144 pairs 77.3 / 77.1, 256 84.7 /
+// 90.9). Past 128 pairs two workgroups share a CU and the gain is gone, so the
+// line lies there, and at T > 1. Four workgroups of 16 rows took the same time
+// up to 128 pairs; without the staging waves, whose work the eight then share,
+// 54 us at 36 pairs and T = 256.
 constexpr int kRows = 32;
 constexpr int kRowsBlock = 16 * kRows + 256;
 template <typename Tin>
@@ -715,7 +723,7 @@ hipError_t launch_infer_t(const InferDesc& d, hipStream_t stream) {
   const dim3 grid(d.H, d.Ba, 1), block(kThreads, 1, 1);
   if (d.T == 1)
     hipLaunchKernelGGL((wkv7_infer_kernel<Tin, 1>), grid, block, 0, stream, p);
-  else if ((int64_t)d.Ba * d.H <= 256)   // its comment has both sides' times
+  else if ((int64_t)d.Ba * d.H <= 128)   // its comment has both sides' times
     hipLaunchKernelGGL(wkv7_infer_rows_kernel<Tin>, dim3(d.H, d.Ba, kHead / kRows), dim3(kRowsBlock), 0, stream, p);
   else
     hipLaunchKernelGGL((wkv7_infer_kernel<Tin, 16>), grid, block, 0, stream, p);
