@@ -303,12 +303,19 @@ __global__ __launch_bounds__(64 * prompt_waves(kSplit)) void wkv7_infer_bf16_pro
 
 }  // namespace
 
-// A CU's registers hold one workgroup, so past 256 pairs they
-// queue: T = 256, us, here (64 rows a workgroup) against the one-wave kernel:
-// 256 pairs 239 / 687, 512 pairs 454 / 702, 768 pairs 678 / 700, 1024 pairs
-// 903 / 696 (T = 8: 16 / 25, 23 / 26, 32 / 26, 42 / 27).
+// A CU's registers hold one workgroup, so past 256 pairs they queue. us, the
+// one-wave kernel and this one:
+//          T = 1       T = 2       T = 4        T = 5        T = 8        T = 16       T = 256
+//   12     5.4 / 5.1   8.0 / 5.8   13.3 / 7.0   16.1 / 7.7   24.0 / 9.6   45.1 / 15.0  679 / 173
+//   256    5.7 / 5.9   8.4 / 6.7   13.6 / 8.5   16.6 / 9.5   24.5 / 11.9  45.4 / 19.2  684 / 229
+//   288    5.8 / 9.2   8.6 / 10.9  14.1 / 14.4  16.9 / 16.4  25.1 / 21.3  47.2 / 35.0  701 / 446
+//   512    6.1 / 9.7   9.0 / 11.5  14.4 / 14.8  17.4 / 16.7  25.5 / 21.8  47.7 / 35.8  701 / 451
+//   576    6.2 / 13.0  9.1 / 15.9  14.4 / 21.0  17.3 / 23.6  25.4 / 31.1  47.5 / 51.9  701 / 668
+// (pairs to the left). One step, where at most 6% are to be had and only up to
+// 128 pairs, stays on the one-wave kernel.
 bool infer_prompt_preferred(const InferDesc& d) {
-  return d.state_dtype == Dtype::BF16 && d.T > 1 && (int64_t)d.Ba * d.H <= 512;
+  const int64_t pairs = (int64_t)d.Ba * d.H;
+  return d.state_dtype == Dtype::BF16 && (d.T > 4 ? pairs <= 512 : d.T > 1 && pairs <= 256);
 }
 
 hipError_t launch_infer_prompt(const InferDesc& d, hipStream_t stream) {

@@ -31,9 +31,11 @@ def _mask(kind, rows, T, rng):
     (1, 2, 1, None), (2, 3, 2, None), (1, 4, 3, "holes"), (3, 5, 2, "edges"), (2, 8, 1, "left"),
     (3, 63, 2, "holes"), (2, 64, 3, "left"), (3, 65, 1, "edges"), (2, 130, 2, "left"),
     (3, 200, 2, "holes"),
-    # 128 and 129 pairs (rows of a pair over two workgroups, over one), 512 and
-    # 513 (the last that runs here, the first that does not)
+    # 128 and 129 pairs (rows of a pair over two workgroups, over one); up to four
+    # steps 256 and 257 (the last that run here, the first that do not), from
+    # five on 512 and 513
     (32, 4, 4, "holes"), (43, 4, 3, None), (43, 9, 3, "left"), (128, 4, 4, "left"), (171, 3, 3, "holes"),
+    (64, 4, 4, "left"), (257, 4, 1, None), (128, 5, 4, "left"), (171, 5, 3, "holes"),
 ])
 def test_prompts_equal_the_oracle(oracle, rows, T, H, mask):
     announce("bf16 prompt", rows, T, H, mask)
