@@ -104,12 +104,14 @@ class KernelOutput:
 
 
 # --------------------------------------------------------------------- helpers
+_DTYPE_CODES = {torch.float32: _native.DTYPE_F32, torch.bfloat16: _native.DTYPE_BF16}
+
+
 def _dtype_code(t: torch.Tensor) -> int:
-    if t.dtype == torch.float32:
-        return _native.DTYPE_F32
-    if t.dtype == torch.bfloat16:
-        return _native.DTYPE_BF16
-    raise TypeError(f"WKV7 operands must be float32 or bfloat16, got {t.dtype}")
+    code = _DTYPE_CODES.get(t.dtype)
+    if code is None:
+        raise TypeError(f"WKV7 operands must be float32 or bfloat16, got {t.dtype}")
+    return code
 
 
 def _ptr(t: Optional[torch.Tensor]):
@@ -229,11 +231,12 @@ def _forward(w, r, k, v, a, b, initial_state, chunk_len, use_initial_state, retu
     output = torch.empty_like(w)
     final_state = (torch.empty((B, H, N, N), dtype=torch.float32, device=dev)
                    if return_final_state else None)
-    ws, nbytes = _workspace("wkv7_forward_workspace_bytes", B, T, H, N, chunk_len,
-                            _dtype_code(w), options, dev)
+    code = _dtype_code(w)
+    ws, nbytes = _workspace("wkv7_forward_workspace_bytes", B, T, H, N, chunk_len, code, options,
+                            dev)
     end = _mark("forward", dev)
     _native.call("wkv7_forward_ws", _ptr(w), _ptr(r), _ptr(k), _ptr(v), _ptr(a), _ptr(b),
-                 _ptr(s0), B, T, H, N, chunk_len, _dtype_code(w), int(use_initial_state),
+                 _ptr(s0), B, T, H, N, chunk_len, code, int(use_initial_state),
                  int(return_final_state), _ptr(state), _ptr(removal_state), _ptr(output),
                  _ptr(final_state), _native.options_ref(options), _ptr(ws), nbytes,
                  _stream(dev))
@@ -253,12 +256,13 @@ def _backward(w, r, k, v, a, b, state, removal_state, output_grad, final_state_g
     grads = [torch.empty_like(w) for _ in range(6)]
     ds0 = (torch.empty((B, H, N, N), dtype=torch.float32, device=dev)
            if write_initial_state_grad else None)
-    ws, nbytes = _workspace("wkv7_backward_workspace_bytes", B, T, H, N, chunk_len,
-                            _dtype_code(w), options, dev)
+    code = _dtype_code(w)
+    ws, nbytes = _workspace("wkv7_backward_workspace_bytes", B, T, H, N, chunk_len, code, options,
+                            dev)
     end = _mark("backward", dev)
     _native.call("wkv7_backward_ws", _ptr(w), _ptr(r), _ptr(k), _ptr(v), _ptr(a), _ptr(b),
                  _ptr(state), _ptr(removal_state), _ptr(output_grad), _ptr(dsT),
-                 B, T, H, N, chunk_len, _dtype_code(w), int(use_final_state_grad),
+                 B, T, H, N, chunk_len, code, int(use_final_state_grad),
                  int(write_initial_state_grad), *(_ptr(g) for g in grads), _ptr(ds0),
                  _native.options_ref(options), _ptr(ws), nbytes, _stream(dev))
     _close(end, dev)
