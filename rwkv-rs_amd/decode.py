@@ -23,7 +23,16 @@ import torch.nn as nn
 from . import _native
 
 MAX_ROWS = 64        # RWKV_DECODE_MAX_ROWS
-MAX_DIM = 8192       # RWKV_DECODE_MAX_DIM
+# The kernels take C up to RWKV_DECODE_MAX_DIM (8192), but they read the fp32
+# weights on every step, and a loop inside one autocast context has the modules
+# cast them once and read half as much. us a step, such a loop through the
+# modules and here, 1 / 17 / 64 sequences: C = 2560, 4 cells 2643 / 535, 2684 / 674,
+# 2653 / 1075; C = 4096, 3 cells 1937 / 632, 1952 / 772, 1953 / 1268; C = 6400, 2
+# cells 1337 / 1067, 1363 / 1308, 1355 / 2168; C = 8192, 2 cells 1369 / 1437, 1468 /
+# 1738, 1601 / 2878. (Replayed from a graph that holds no casts the modules take
+# 1124 at C = 4096 and 64 sequences against 1252, elsewhere up to 4096 they are
+# slower; with a context a step, 2157 and more at C = 4096.)
+MAX_DIM = 4096
 
 
 def _plain(module, cls) -> bool:

@@ -253,3 +253,25 @@ def test_a_state_without_elapsed_t_is_refused_as_by_the_modules():
     st.elapsed_t = None
     with pytest.raises(ValueError, match="elapsed_t required"):
         _infer(model, torch.zeros(2, 1, dtype=torch.long, device=DEV), torch.arange(2, device=DEV), st)
+
+
+def _wide_model(heads, cells=1, vocab=33):
+    m = load_pkg().model
+    with torch.device(DEV):
+        model = m.AutoRegressiveModel(vocab, cells, heads * 64, heads, 64, wkv7_dtype=torch.bfloat16,
+                                      neighbor_ops="hip")
+    # products of the size that std 0.2 gives at two heads
+    return model.init_random(0.2 * (2 / heads) ** 0.5, torch.Generator(DEV).manual_seed(1))
+
+
+@pytest.mark.parametrize("heads,fused", [(64, True), (65, False)])
+def test_the_widest_model_of_the_fused_step(monkeypatch, heads, fused):
+    announce("decode step, where the widths end", heads)
+    decode = load_pkg().decode
+    model = _wide_model(heads)
+    taken = []
+    real = decode.step
+    monkeypatch.setattr(decode, "step", lambda *x: taken.append(real(*x)) or taken[-1])
+    ids, toks = torch.arange(2, device=DEV), torch.arange(2, device=DEV).reshape(2, 1)
+    _infer(model, toks, ids, _state(model, 2, torch.bfloat16, 1))
+    assert (taken[0] is not None) == fused
