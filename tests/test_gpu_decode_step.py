@@ -275,3 +275,80 @@ def test_the_widest_model_of_the_fused_step(monkeypatch, heads, fused):
     ids, toks = torch.arange(2, device=DEV), torch.arange(2, device=DEV).reshape(2, 1)
     _infer(model, toks, ids, _state(model, 2, torch.bfloat16, 1))
     assert (taken[0] is not None) == fused
+
+
+@pytest.mark.parametrize("heads,rows,state_dtype", [
+    (16, 5, torch.bfloat16),                              # C = 1024: the last of four channels a thread
+    (17, 3, torch.bfloat16), (31, 18, torch.float32), (32, 33, torch.bfloat16),     # eight: 1088 .. 2048
+    (33, 2, torch.float32), (64, 17, torch.bfloat16), (128, 3, torch.bfloat16),     # 32: 2112 .. 8192
+])
+def test_a_fused_step_of_a_wide_model_matches_the_modules(monkeypatch, heads, rows, state_dtype):
+    # each instance of the norms, and the products' rounds over K = C and 4 C;
+    # the kernels' widest is wider than what infer sends to them
+    announce("decode step, wide", heads, rows, str(state_dtype))
+    decode = load_pkg().decode
+    monkeypatch.setattr(decode, "MAX_DIM", 8192)
+    model = _wide_model(heads)
+    ids, toks = torch.arange(rows, device=DEV), torch.arange(rows, device=DEV).reshape(rows, 1) % 33
+    a, b = _state(model, rows, state_dtype, 7), _state(model, rows, state_dtype, 7)
+    taken = []
+    real = decode.step
+    monkeypatch.setattr(decode, "step", lambda *x: taken.append(real(*x)) or taken[-1])
+    got = _infer(model, toks, ids, a)
+    monkeypatch.setattr(decode, "step", lambda *x: None)
+    want = _infer(model, toks, ids, b)
+    assert taken[0] is not None and _err(got, want) < 1e-2
+    for x, y in zip(a.state + a.shift_time + a.shift_channel, b.state + b.shift_time + b.shift_channel):
+        assert _err(x, y) < 1e-2
+
+
+def test_a_captured_step_replays_and_streams_do_not_share():
+    # the workspace and the residual stream come from the capture's pool; eager
+    # steps of another size between the replays, and two streams at once
+    announce("decode step in a graph and on two streams")
+    model = _model(3)
+    ids, toks = torch.arange(5, device=DEV), torch.arange(5, device=DEV).reshape(5, 1)
+    start = _state(model, 6, torch.bfloat16, 1)
+    st = _state(model, 6, torch.bfloat16, 1)
+    lists = ("state", "shift_time", "shift_channel")
+
+    def reset(s, to=start):
+        for n in lists:
+            for x, y in zip(getattr(s, n), getattr(to, n)):
+                x.copy_(y)
+    eager = _state(model, 6, torch.bfloat16, 1)
+    want = _infer(model, toks, ids, eager).clone()
+    # the shifts' next buffers replace those of infer_state, so a captured step
+    # starts from the tensors that it was captured with
+    held = {n: list(getattr(st, n)) for n in lists}
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        _infer(model, toks, ids, _state(model, 6, torch.bfloat16, 1))
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = _infer(model, toks, ids, st)
+    out = {n: list(getattr(st, n)) for n in lists}
+    for _ in range(3):
+        got.zero_()
+        for n in lists:
+            for x, y in zip(held[n], getattr(start, n)):
+                x.copy_(y)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
+        for n in lists:
+            assert all(torch.equal(x, y) for x, y in zip(out[n], getattr(eager, n)))
+        _infer(model, toks[:2], ids[:2], _state(model, 6, torch.float32, 2))
+    streams, got = [torch.cuda.Stream() for _ in range(2)], [[], []]
+    sts = [_state(model, 6, torch.bfloat16, 1) for _ in range(2)]
+    torch.cuda.synchronize()
+    for _ in range(4):
+        for i, stream in enumerate(streams):
+            with torch.cuda.stream(stream):
+                reset(sts[i])
+                got[i].append(_infer(model, toks, ids, sts[i]))
+    torch.cuda.synchronize()
+    assert all(torch.equal(x, want) for g in got for x in g)
