@@ -1,7 +1,5 @@
-"""CPU-only checks of the C ABI (include/wkv7.h, include/rwkv_neighbors.h,
-include/rwkv_lm_loss.h):
-the library loads, exports
-every declared entry point, and rejects bad calls on the host with the right
+"""CPU-only checks of the C ABI (the headers under include/): the library
+loads, exports every declared entry point, and rejects bad calls on the host with the right
 status before any HIP call. No kernel is launched here: every call either
 fails validation or has nothing to do."""
 
@@ -45,6 +43,15 @@ def test_library_exports_every_declared_symbol(native):
     for name in declared:
         assert hasattr(lib, name), name
     assert set(declared) == set(native.EXPORTS)
+
+
+@pytest.mark.parametrize("header,prefix,exports,count", [
+    ("wkv7_segments.h", "wkv7_", "SEGMENT_EXPORTS", 4), ("rwkv_decode.h", "rwkv_", "DECODE_EXPORTS", 3)])
+def test_library_exports_what_the_other_headers_declare(native, header, prefix, exports, count):
+    declared = declared_functions(os.path.join(REPO, "include", header), prefix)
+    assert len(declared) == count and set(declared) == set(getattr(native, exports))
+    for name in declared:
+        assert hasattr(native.lib(), name) and name in native._SIGNATURES, name
 
 
 def test_version_and_strings(native):

@@ -185,3 +185,44 @@ def test_a_given_up_wait_poisons_the_whole_pair(wk, dtype):
     assert [fwd_faults, bwd_faults] == hit and hit[0] > 0
     again = wk.wkv7_statepass_forward(*ins, s0, 16)
     assert wk.take_faults() == 0 and torch.equal(again.output, good.output)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("case", [(1, 32 * 40, 4, 32, BF16), (2, 32 * 20, 8, 32, BF16), (1, 32 * 41, 4, 32, F32),
+                                  (1, 2048 + 16 * 5, 3, 16, F32), (1, 2048 + 16 * 5, 3, 16, BF16)])
+def test_backward_from_the_segmented_forwards_checkpoints(wk, monkeypatch, case):
+    # at chunk_len 32 the backward rebuilds states from the checkpoints, which
+    # multiplies their deviation by about 1.35 a step (120 over the 16 between
+    # them); the two forwards' checkpoints are 1e-8 apart at fp32 products, so
+    # their 1e-6 stays inside the gradients' bar
+    B, T, H, chunk, dtype = case
+    announce("segments, forward's checkpoints into the backward", case)
+    bf16 = dtype == BF16
+    td = torch.bfloat16 if bf16 else torch.float32
+    d = load_pkg().synthetic.make_inputs(B, T, H, 64, seed=T + H, s0_std=0.5, bf16=bf16)
+    ins = [to_dev(d[n], td) for n in NAMES]
+    s0, dy = to_dev(d["s0"]), to_dev(d["dy"], td)
+    dsT = 0.3 * torch.randn(B, H, 64, 64, device="cuda", generator=torch.Generator("cuda").manual_seed(T))
+    assert _segments("forward", B, T, H, chunk, dtype) > 1 and _segments("backward", B, T, H, chunk, dtype) > 1
+
+    def chain():
+        f = wk.wkv7_statepass_forward(*ins, s0, chunk)
+        return wk.wkv7_statepass_backward(*ins, f.state, f.removal_state, dy, dsT, chunk)
+    cut = chain()
+    native = wk._native
+
+    class OnePiece:
+        def __getattr__(self, name):
+            return getattr(native, name)
+
+        @staticmethod
+        def call(name, *args):
+            _in_one_piece(name.replace("_ws", "_ex"), args)
+    with monkeypatch.context() as m:
+        m.setattr(wk, "_native", OnePiece())
+        one = chain()
+    torch.cuda.synchronize()
+    for name in GRAD_NAMES + ("initial_state_grad",):
+        err = rel_l2(to_np(getattr(cut, name)), to_np(getattr(one, name)))
+        print(name, err, flush=True)
+        assert err <= ((1.2e-5 if name == "initial_state_grad" else 4e-4) if bf16 else 2e-5), (name, err)
