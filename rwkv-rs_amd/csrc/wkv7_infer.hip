@@ -266,7 +266,7 @@ __global__ __launch_bounds__(kRowsBlock) void wkv7_infer_rows_kernel(InferParams
       }
       lds_barrier();
     }
-    if (ntiles > 0) outputs(ntiles - 1);
+    outputs(ntiles - 1);   // T > 0: launch_infer launches nothing else
     return;
   }
 
