@@ -21,7 +21,8 @@
 extern "C" {
 #endif
 
-/* Sequences a call may have, and the widest embedding (a row is held in LDS). */
+/* Sequences a call may have (four tiles of the 16 rows of a matrix product), and
+ * the widest embedding (a norm's 256 threads hold a row, 32 channels each). */
 #define RWKV_DECODE_MAX_ROWS 64
 #define RWKV_DECODE_MAX_DIM 8192
 

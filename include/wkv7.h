@@ -116,9 +116,10 @@ typedef enum wkv7_status {
   WKV7_ERR_HIP = 9,          /* the kernel launch failed */
   WKV7_ERR_SCRATCH_LIMIT = 10, /* the call needs more than the library's fixed
                                  scratch array (the _noalloc entry points) */
-  WKV7_ERR_HANDOVER = 11      /* a chunked-forward launch gave up an internal
-                                 wait; its outputs were poisoned with NaN
-                                 (reported by wkv7_take_faults) */
+  WKV7_ERR_HANDOVER = 11      /* a chunked forward, or a call cut into
+                                 segments, gave up an internal wait; its
+                                 outputs were poisoned with NaN (reported by
+                                 wkv7_take_faults) */
 } wkv7_status;
 
 typedef enum wkv7_dtype { WKV7_DTYPE_F32 = 0, WKV7_DTYPE_BF16 = 1 } wkv7_dtype;
@@ -179,8 +180,8 @@ int wkv7_backward(const void *weight_decay, const void *receptance,
  * the arithmetic of each family is described at the top
  * of this file. WKV7_KERNELS_STEP runs the step kernels for every case (to
  * compare the families on one input). handover_spin_limit bounds the polls
- * of each hand-over wait inside the chunked forwards (0 = the default,
- * about 0.1 s); it exists so that tests can force the fault path below.
+ * of each hand-over wait inside the chunked forwards and the first pass of
+ * calls cut into segments (0 = the default, about 0.1 s); it exists so that tests can force the fault path below.
  * options may be NULL (all defaults).
  * ------------------------------------------------------------------------- */
 typedef enum wkv7_kernels { WKV7_KERNELS_AUTO = 0, WKV7_KERNELS_STEP = 1 } wkv7_kernels;
@@ -212,17 +213,17 @@ int wkv7_backward_ex(const void *weight_decay, const void *receptance,
                      float *initial_state_grad, const wkv7_options *options,
                      void *stream);
 
-/* Hand-over faults of the chunked forwards (bf16 and fp32 operands). Their
+/* Hand-over faults of the chunked forwards (bf16 and fp32 operands) and of
+ * calls cut into segments (wkv7_segments.h), forward and backward. Their
  * producer and consumer waves pass chunks through LDS flags with bounded
- * waits. A wait that gives up
- * (which a correct kernel never does) makes the launch overwrite every output
- * of that (batch, head) -- output, removal_state, the checkpoints, the final
- * state -- with NaN, and adds one to a counter on the device. So does a call
- * cut into segments, whichever of its passes gave up (a backward's first pass
- * has such waits too: its gradients then). No counterpart in the reference. wkv7_take_faults waits for `stream`, stores in *count the
- * number of such events on the current device since the previous call,
- * resets the counter, and returns WKV7_ERR_HANDOVER if *count > 0 (WKV7_OK
- * otherwise). Calls on one device must not overlap. */
+ * waits. A wait that gives up (which a correct kernel never does) makes the
+ * call overwrite every output of that (batch, head) with NaN -- a forward's
+ * output, removal_state, checkpoints and final state, a backward's gradients
+ * -- and adds one to a counter on the device, whichever pass and segment it
+ * was. No counterpart in the reference. wkv7_take_faults waits for `stream`,
+ * stores in *count the number of such (batch, head)s on the current device
+ * since the previous call, resets the counter, and returns WKV7_ERR_HANDOVER
+ * if *count > 0 (WKV7_OK otherwise). Calls on one device must not overlap. */
 int wkv7_take_faults(void *stream, uint32_t *count);
 
 /* Device self-test of two bf16 building blocks, run exactly as the kernels

@@ -12,9 +12,10 @@
 //   norm + token shift + mix, key product + relu^2, value product + residual
 // The weights are read as they are stored, fp32, and rounded to bf16 in
 // registers, so no bf16 copy of them is made or kept. At 12 cells, C = 768, 8
-// sequences, vocabulary 65536, a step took 8,900 us through the modules and
-// takes 790 so (kernel time 4.0 ms and 0.78 ms, of which the head's 201 MB of
-// weights are 45 us; the rest is the launches' own latency, 3-9 us each).
+// sequences, vocabulary 65536, a step took 9,150 us through the modules and
+// takes 835 so. Its kernels sum to 694 us, of which the head's 201 MB of
+// weights are 48; the rest is each launch's own latency, 3-9 us (profiles/
+// rwkv7_0.1b_decode_step_kernel_stats.md).
 #include "decode_launch.hpp"
 
 #include "neighbors_device.hpp"
@@ -59,7 +60,11 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
 // copies slot s unless a row writes it. A thread holds kChannels channels, and
 // loads all that they need before the first sum, so that the sums wait for one
 // memory latency (at C = 768, six mixes / one: 5.2 / 5.7 us a launch with the
-// row in LDS and the parameters loaded after the sums, 4.2 / 3.3 us so).
+// row in LDS and the parameters loaded after the sums, 4.2 / 3.3 us so). Six
+// mixes / one, us a launch with 4 channels a thread: C = 1024 4.2 / 3.4; with 8:
+// 1088 4.9 / 3.6, 2048 5.0 / 3.8; with 32, most of a wave's registers and one
+// wave a SIMD: 2112 7.5 / 4.9, 4096 8.5 / 5.7, beside 87 us of products a cell
+// at 2112 and 194 at 4096.
 template <int NM, int kChannels>
 __global__ __launch_bounds__(256) void norm_mix_kernel(const NormArgs a) {
   __shared__ float red[4];

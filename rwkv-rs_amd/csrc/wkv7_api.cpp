@@ -188,7 +188,7 @@ const char* wkv7_strerror(int status) {
       return "invalid flag value, flag/pointer mismatch, or dither asked for an fp32 state";
     case WKV7_ERR_HIP: return "HIP kernel launch failed";
     case WKV7_ERR_HANDOVER:
-      return "a chunked forward gave up an internal hand-over wait; its outputs are NaN";
+      return "a chunked forward, or a call cut into segments, gave up an internal hand-over wait; its outputs are NaN";
     case WKV7_ERR_SCRATCH_LIMIT:
       return "the call needs more scratch memory than the library's fixed device array holds";
     default: return "unknown wkv7 status";

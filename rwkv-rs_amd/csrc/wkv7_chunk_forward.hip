@@ -46,8 +46,8 @@ constexpr int kBlock = 64 * kWaves;
 constexpr int kVecs = 6;                  // staged inputs: x, r, k, a, b, v
 enum { S_X, S_R, S_K, S_A, S_B, S_V };
 constexpr int kPieces = kVecs * kL * 8 / 64;   // 16-byte loads per prep lane and chunk
-// hand-over faults of the chunked forwards on this device since the host
-// last took them, and the value the last take read
+// hand-over faults of chunked forwards and segmented calls on this device since
+// the host last took them, and the value the last take read
 __device__ unsigned int handover_faults;
 __device__ unsigned int handover_faults_taken;
 

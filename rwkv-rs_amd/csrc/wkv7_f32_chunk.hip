@@ -187,7 +187,7 @@ struct F32FwdParams {
   float* sa;                  // [B,T,H,64]
   Tin* y;                     // [B,T,H,64]
   float* sT;                  // [B,H,64,64] or null
-  unsigned int* faults;       // the chunked forwards' hand-over fault counter
+  unsigned int* faults;       // the hand-over fault counter
   int T, H, C;
   int cps;                    // chunks per workgroup: all of a sequence's, or a segment's
   const float* bound;         // segment g > 0 of [B,H,G,64,64]: its start state

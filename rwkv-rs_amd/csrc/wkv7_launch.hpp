@@ -11,7 +11,7 @@ constexpr int kHeadSize = 64;   // the kernels are specialised for N = 64
 
 enum class Dtype : int { F32 = 0, BF16 = 1 };
 
-// kernel family (WKV7_KERNELS_*) and the chunked forward's hand-over bound
+// kernel family (WKV7_KERNELS_*) and the hand-over bound
 struct KernelChoice {
   bool step_only = false;       // WKV7_KERNELS_STEP
   uint32_t spin_limit = 0;      // 0 = default
@@ -107,8 +107,8 @@ hipError_t launch_segment_poison(const ForwardDesc& d, hipStream_t stream);
 // asked for the step kernels (KernelChoice::step_only).
 bool chunk_forward_supported(const ForwardDesc& d);
 hipError_t launch_forward_chunked(const ForwardDesc& d, hipStream_t stream);
-// the chunked forwards' hand-over fault counter on the current device: read
-// and reset on `stream`, then wait for it
+// the hand-over fault counter of chunked forwards and segmented calls on the
+// current device: read and reset on `stream`, then wait for it
 hipError_t take_handover_faults(hipStream_t stream, uint32_t* count);
 // that counter's device address on the current device
 hipError_t handover_fault_counter(unsigned int** counter);

@@ -714,8 +714,9 @@ def train_step(model: AutoRegressiveModel, optimizer, inputs, targets, kernel=No
     """One pretrain step: forward, loss, backward, optimizer update
     (model.rs:316-324). Returns the detached loss. With ``check_faults`` the
     step ends by waiting for the device and raising ``Wkv7Error`` if a
-    chunked forward of the step gave up a hand-over wait (its outputs, and so
-    the loss, are then NaN); without it the step stays asynchronous and the
+    chunked forward of the step, or a call of it cut into segments, gave up a
+    hand-over wait (its outputs, and so the loss or the gradients, are then
+    NaN); without it the step stays asynchronous and the
     caller polls ``wkv7.check_faults`` where it synchronises anyway."""
     device_type = inputs.device.type
     with torch.autocast(device_type, dtype=torch.bfloat16, enabled=autocast):

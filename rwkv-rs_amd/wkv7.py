@@ -297,8 +297,9 @@ def wkv7_backward_ex(weight_decay, receptance, key, value, removal, replacement,
 
 def take_faults(device=None) -> int:
     """wkv7_take_faults: waits for the current stream, resets the device's
-    counter and returns the number of chunked-forward launches on the device
-    that gave up a hand-over wait since the last call (their outputs are NaN).
+    counter and returns the number of (batch, head) pairs on the device whose
+    chunked forward, or segmented forward or backward, gave up a hand-over wait
+    since the last call (their outputs are NaN).
     Other failures of the call raise Wkv7Error."""
     import ctypes
     dev = torch.device("cuda", torch.cuda.current_device()) if device is None else device
@@ -310,9 +311,9 @@ def take_faults(device=None) -> int:
 
 
 def check_faults(device=None) -> None:
-    """Raises Wkv7Error (WKV7_ERR_HANDOVER) when a chunked forward on the
-    device gave up a hand-over wait since the last take_faults/check_faults,
-    i.e. when some of the outputs computed since then are NaN by that cause.
+    """Raises Wkv7Error (WKV7_ERR_HANDOVER) when a chunked forward, or a call
+    cut into segments, on the device gave up a hand-over wait since the last
+    take_faults/check_faults, i.e. when some of the outputs computed since then are NaN by that cause.
     Waits for the current stream: call it where the caller synchronises
     anyway (the end of a step, a logged loss), not inside a captured graph."""
     n = take_faults(device)
