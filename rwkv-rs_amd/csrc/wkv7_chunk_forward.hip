@@ -75,9 +75,10 @@ struct FwdChunkParams {
   bf16_t* y;
   float* sT;
   int T, H;
-  int cps;                   // chunks per workgroup: all of a sequence's, or a segment's
+  // segmented calls only:
+  int cps;                   // chunks per segment
   const float* bound;        // segment g > 0 of [B,H,G,64,64]: its start state
-  int* fault;                // [B,H,G] (segmented calls only)
+  int* fault;                // [B,H,G]
   uint32_t spin_limit;       // polls per hand-over wait (> 0)
 };
 
@@ -286,7 +287,8 @@ __device__ __forceinline__ uint4 load_stream(const uint4* q) {
 }
 
 // Grid (H, B, G): workgroup (h, b, g) runs segment g of the sequence, chunks
-// g cps .. (a sequence in one piece is its only segment).
+// g cps ..
+template <Start kStart>
 __global__ __launch_bounds__(kBlock, 1) void wkv7_fwd_chunk_kernel(const FwdChunkParams p) {
   __shared__ ChunkOps ops[kSlots];
   __shared__ __attribute__((aligned(16))) PrepLds prep[kSlots];
@@ -297,12 +299,13 @@ __global__ __launch_bounds__(kBlock, 1) void wkv7_fwd_chunk_kernel(const FwdChun
   const int h = blockIdx.x, b = blockIdx.y, H = p.H, T = p.T;
   const int64_t bh = (int64_t)b * H + h;
   const int64_t tstride = (int64_t)H * kHead;              // elements per step
-  const int g = blockIdx.z, total = T / kL;
-  const int c0 = g * p.cps, nchunks = min(p.cps, total - c0);   // this segment's chunks
+  constexpr bool kSeg = kStart == Start::kSegment;
+  const int g = kSeg ? blockIdx.z : 0, total = T / kL;
+  const int c0 = kSeg ? g * p.cps : 0, nchunks = kSeg ? min(p.cps, total - c0) : total;   // this segment's chunks
   // step 0 of (b, h)'s segment
   const int64_t tok0 = (((int64_t)b * T + (int64_t)kL * c0) * H + h) * kHead;
-  const float* const s0 = g > 0 ? p.bound + (bh * gridDim.z + g) * (kHead * kHead)
-                        : p.s0 ? p.s0 + bh * (kHead * kHead) : nullptr;
+  const float* const s0 = start_state<kStart>(p.s0, p.bound, bh, g);
+  const bool has_s0 = kStart == Start::kGiven || (kSeg && s0);
 
   if (tid < kSlots) flags.ready[tid] = -1;
   if (tid == 0) flags.fault = 0;
@@ -354,7 +357,7 @@ __global__ __launch_bounds__(kBlock, 1) void wkv7_fwd_chunk_kernel(const FwdChun
     f32x4 S[4];
 #pragma unroll
     for (int ib = 0; ib < 4; ++ib) {
-      if (s0)
+      if (has_s0)
         S[ib] = *reinterpret_cast<const f32x4*>(s0 + jcol * kHead + 16 * ib + 4 * qd);
       else
         S[ib] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -417,7 +420,7 @@ __global__ __launch_bounds__(kBlock, 1) void wkv7_fwd_chunk_kernel(const FwdChun
     }
     if (nchunks > 0) store_ckpt(nchunks - 1, S);
 
-    if (p.sT && c0 + nchunks == total) {
+    if (p.sT && (!kSeg || c0 + nchunks == total)) {
 #pragma unroll
       for (int ib = 0; ib < 4; ++ib)
         *reinterpret_cast<f32x4*>(p.sT + bh * (kHead * kHead) + jcol * kHead + 16 * ib + 4 * qd) = S[ib];
@@ -429,7 +432,7 @@ __global__ __launch_bounds__(kBlock, 1) void wkv7_fwd_chunk_kernel(const FwdChun
   // event is counted for the host; a segment leaves its word for the kernel
   // that does this after all segments
   __syncthreads();
-  if (p.fault) {
+  if (kSeg) {
     if (tid == 0 && lds_load_flag(&flags.fault)) p.fault[bh * gridDim.z + g] = 1;
   } else if (lds_load_flag(&flags.fault)) {
     poison_forward(p.y, p.sa, p.ckpt, p.sT, b, h, H, T, total, tid, kBlock);
@@ -471,14 +474,16 @@ hipError_t launch_forward_chunked(const ForwardDesc& d, hipStream_t stream) {
   p.sT = d.sT;
   p.T = d.T;
   p.H = d.H;
-  p.cps = d.seg.G > 1 ? d.seg.cps : d.T / kL;
+  p.cps = d.seg.cps;
   p.bound = d.seg.bound;
-  p.fault = d.seg.G > 1 ? d.seg.fault : nullptr;
+  p.fault = d.seg.fault;
   p.spin_limit = d.kc.spin_limit ? d.kc.spin_limit : kSpinLimit;
   const dim3 grid(d.H, d.B, d.seg.G), block(kBlock, 1, 1);
   if (d.seg.G > 1)
     if (hipError_t e = launch_segment_bounds(d, stream)) return e;
-  hipLaunchKernelGGL(wkv7_fwd_chunk_kernel, grid, block, 0, stream, p);
+  auto* const kernel = d.seg.G > 1 ? wkv7_fwd_chunk_kernel<Start::kSegment>
+                       : d.s0 ? wkv7_fwd_chunk_kernel<Start::kGiven> : wkv7_fwd_chunk_kernel<Start::kZero>;
+  hipLaunchKernelGGL(kernel, grid, block, 0, stream, p);
   hipError_t e = hipGetLastError();
   return e == hipSuccess && d.seg.G > 1 ? launch_segment_poison(d, stream) : e;
 }

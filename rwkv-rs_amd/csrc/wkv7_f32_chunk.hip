@@ -189,9 +189,10 @@ struct F32FwdParams {
   float* sT;                  // [B,H,64,64] or null
   unsigned int* faults;       // the hand-over fault counter
   int T, H, C;
-  int cps;                    // chunks per workgroup: all of a sequence's, or a segment's
+  // segmented calls only:
+  int cps;                    // chunks per segment
   const float* bound;         // segment g > 0 of [B,H,G,64,64]: its start state
-  int* fault;                 // [B,H,G] (segmented calls only)
+  int* fault;                 // [B,H,G]
   uint32_t spin_limit;        // polls per hand-over wait (> 0)
 };
 
@@ -229,9 +230,8 @@ __device__ __forceinline__ f32x4 col_frag4(const Tin* base, int64_t tstride, int
 }
 
 // Grid (H, B, G): workgroup (h, b, g) runs segment g of the sequence, chunks
-// g cps .. (a sequence in one piece is its only segment); a segment is a whole
-// number of checkpoint intervals.
-template <typename Tin>
+// g cps ..; a segment is a whole number of checkpoint intervals.
+template <typename Tin, Start kStart>
 __global__ __launch_bounds__(kBlock, 1) void wkv7_fwd_f32_chunk_kernel(const F32FwdParams<Tin> p) {
   __shared__ F32ChunkOps ops[kSlots];
   __shared__ F32PrepLds prep[kSlots];
@@ -244,10 +244,12 @@ __global__ __launch_bounds__(kBlock, 1) void wkv7_fwd_f32_chunk_kernel(const F32
   const int h = blockIdx.x, b = blockIdx.y, H = p.H, T = p.T;
   const int64_t bh = (int64_t)b * H + h;
   const int64_t tstride = (int64_t)H * kHead;
-  const int g = blockIdx.z, c0 = g * p.cps, nchunks = min(p.cps, T / kL - c0);   // this segment's chunks
+  constexpr bool kSeg = kStart == Start::kSegment;
+  const int g = kSeg ? blockIdx.z : 0, c0 = kSeg ? g * p.cps : 0;
+  const int nchunks = kSeg ? min(p.cps, T / kL - c0) : T / kL;   // this segment's chunks
   const int64_t tok0 = (((int64_t)b * T + (int64_t)kL * c0) * H + h) * kHead;
-  const float* const s0 = g > 0 ? p.bound + (bh * gridDim.z + g) * (kHead * kHead)
-                        : p.s0 ? p.s0 + bh * (kHead * kHead) : nullptr;
+  const float* const s0 = start_state<kStart>(p.s0, p.bound, bh, g);
+  const bool has_s0 = kStart == Start::kGiven || (kSeg && s0);
   const int per_ckpt = p.C / kL;
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
 
@@ -404,7 +406,7 @@ __global__ __launch_bounds__(kBlock, 1) void wkv7_fwd_f32_chunk_kernel(const F32
 #pragma unroll
     for (int ib = 0; ib < 4; ++ib) {
       // s0 is [value][key]: register r holds key 16 ib + 4 qd + r of value jcol
-      if (s0)
+      if (has_s0)
         S[ib] = *reinterpret_cast<const f32x4*>(s0 + jcol * kHead + 16 * ib + 4 * qd);
       else
         S[ib] = zero;
@@ -473,7 +475,7 @@ __global__ __launch_bounds__(kBlock, 1) void wkv7_fwd_f32_chunk_kernel(const F32
       }
       if ((c + 1) % per_ckpt == 0) store_ckpt((c + 1) / per_ckpt - 1);
     }
-    if (p.sT && c0 + nchunks == T / kL) {
+    if (p.sT && (!kSeg || c0 + nchunks == T / kL)) {
 #pragma unroll
       for (int ib = 0; ib < 4; ++ib)
         *reinterpret_cast<f32x4*>(p.sT + bh * (kHead * kHead) + jcol * kHead + 16 * ib + 4 * qd) = S[ib];
@@ -485,7 +487,7 @@ __global__ __launch_bounds__(kBlock, 1) void wkv7_fwd_f32_chunk_kernel(const F32
   // event is counted for the host; a segment leaves its word for the kernel
   // that does this after all segments
   __syncthreads();
-  if (p.fault) {
+  if (kSeg) {
     if (tid == 0 && lds_load_flag(&flags.fault)) p.fault[bh * gridDim.z + g] = 1;
   } else if (lds_load_flag(&flags.fault)) {
     poison_forward(p.y, p.sa, p.ckpt, p.sT, b, h, H, T, T / p.C, tid, kBlock);
@@ -1180,16 +1182,18 @@ static hipError_t launch_fwd_f32(const ForwardDesc& d, hipStream_t stream) {
   p.H = d.H;
   p.C = d.C;
   p.spin_limit = d.kc.spin_limit ? d.kc.spin_limit : kSpinLimit;
-  p.cps = d.seg.G > 1 ? d.seg.cps : d.T / kL;
+  p.cps = d.seg.cps;
   p.bound = d.seg.bound;
-  p.fault = d.seg.G > 1 ? d.seg.fault : nullptr;
+  p.fault = d.seg.fault;
   // the counter lives in the bf16 forward's code object; its address is
   // looked up on the current device at every launch (a host-side lookup, no
   // stream work, so captured launches replay it as they are)
   hipError_t e = handover_fault_counter(&p.faults);
   if (e != hipSuccess) return e;
   if (d.seg.G > 1 && (e = launch_segment_bounds(d, stream)) != hipSuccess) return e;
-  hipLaunchKernelGGL(wkv7_fwd_f32_chunk_kernel<Tin>, dim3(d.H, d.B, d.seg.G), dim3(kBlock), 0, stream, p);
+  auto* const kernel = d.seg.G > 1 ? wkv7_fwd_f32_chunk_kernel<Tin, Start::kSegment>
+                       : d.s0 ? wkv7_fwd_f32_chunk_kernel<Tin, Start::kGiven> : wkv7_fwd_f32_chunk_kernel<Tin, Start::kZero>;
+  hipLaunchKernelGGL(kernel, dim3(d.H, d.B, d.seg.G), dim3(kBlock), 0, stream, p);
   e = hipGetLastError();
   return e == hipSuccess && d.seg.G > 1 ? launch_segment_poison(d, stream) : e;
 }
