@@ -307,13 +307,15 @@ __device__ __forceinline__ void lds_acquire() {
 // initial state, that one / its own: bf16, T = 64, 8 pairs 10.55 / 10.34, 256
 // pairs 13.80 / 13.63; fp32 18.88 / 18.78 and 23.39 / 23.15; from T = 256 on no
 // difference).
-enum class Start { kZero, kGiven, kSegment };
+namespace start {   // int: kernel names carry the value
+constexpr int kZero = 0, kGiven = 1, kSegment = 2;
+}
 // the start state of segment g, or null for zeros
-template <Start kStart>
+template <int kStart>
 __device__ __forceinline__ const float* start_state(const float* s0, const float* bound, int64_t bh, int g) {
-  if (kStart == Start::kZero) return nullptr;
-  if (kStart == Start::kSegment && g > 0) return bound + (bh * gridDim.z + g) * (kHead * kHead);
-  return kStart == Start::kGiven || s0 ? s0 + bh * (kHead * kHead) : nullptr;
+  if (kStart == start::kZero) return nullptr;
+  if (kStart == start::kSegment && g > 0) return bound + (bh * gridDim.z + g) * (kHead * kHead);
+  return kStart == start::kGiven || s0 ? s0 + bh * (kHead * kHead) : nullptr;
 }
 
 // every output of one (batch, head) of a forward to NaN, by the threads of a

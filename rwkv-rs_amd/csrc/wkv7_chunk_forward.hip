@@ -288,7 +288,7 @@ __device__ __forceinline__ uint4 load_stream(const uint4* q) {
 
 // Grid (H, B, G): workgroup (h, b, g) runs segment g of the sequence, chunks
 // g cps ..
-template <Start kStart>
+template <int kStart>
 __global__ __launch_bounds__(kBlock, 1) void wkv7_fwd_chunk_kernel(const FwdChunkParams p) {
   __shared__ ChunkOps ops[kSlots];
   __shared__ __attribute__((aligned(16))) PrepLds prep[kSlots];
@@ -299,13 +299,13 @@ __global__ __launch_bounds__(kBlock, 1) void wkv7_fwd_chunk_kernel(const FwdChun
   const int h = blockIdx.x, b = blockIdx.y, H = p.H, T = p.T;
   const int64_t bh = (int64_t)b * H + h;
   const int64_t tstride = (int64_t)H * kHead;              // elements per step
-  constexpr bool kSeg = kStart == Start::kSegment;
+  constexpr bool kSeg = kStart == start::kSegment;
   const int g = kSeg ? blockIdx.z : 0, total = T / kL;
   const int c0 = kSeg ? g * p.cps : 0, nchunks = kSeg ? min(p.cps, total - c0) : total;   // this segment's chunks
   // step 0 of (b, h)'s segment
   const int64_t tok0 = (((int64_t)b * T + (int64_t)kL * c0) * H + h) * kHead;
   const float* const s0 = start_state<kStart>(p.s0, p.bound, bh, g);
-  const bool has_s0 = kStart == Start::kGiven || (kSeg && s0);
+  const bool has_s0 = kStart == start::kGiven || (kSeg && s0);
 
   if (tid < kSlots) flags.ready[tid] = -1;
   if (tid == 0) flags.fault = 0;
@@ -481,8 +481,8 @@ hipError_t launch_forward_chunked(const ForwardDesc& d, hipStream_t stream) {
   const dim3 grid(d.H, d.B, d.seg.G), block(kBlock, 1, 1);
   if (d.seg.G > 1)
     if (hipError_t e = launch_segment_bounds(d, stream)) return e;
-  auto* const kernel = d.seg.G > 1 ? wkv7_fwd_chunk_kernel<Start::kSegment>
-                       : d.s0 ? wkv7_fwd_chunk_kernel<Start::kGiven> : wkv7_fwd_chunk_kernel<Start::kZero>;
+  auto* const kernel = d.seg.G > 1 ? wkv7_fwd_chunk_kernel<start::kSegment>
+                       : d.s0 ? wkv7_fwd_chunk_kernel<start::kGiven> : wkv7_fwd_chunk_kernel<start::kZero>;
   hipLaunchKernelGGL(kernel, grid, block, 0, stream, p);
   hipError_t e = hipGetLastError();
   return e == hipSuccess && d.seg.G > 1 ? launch_segment_poison(d, stream) : e;

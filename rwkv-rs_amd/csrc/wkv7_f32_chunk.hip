@@ -231,7 +231,7 @@ __device__ __forceinline__ f32x4 col_frag4(const Tin* base, int64_t tstride, int
 
 // Grid (H, B, G): workgroup (h, b, g) runs segment g of the sequence, chunks
 // g cps ..; a segment is a whole number of checkpoint intervals.
-template <typename Tin, Start kStart>
+template <typename Tin, int kStart>
 __global__ __launch_bounds__(kBlock, 1) void wkv7_fwd_f32_chunk_kernel(const F32FwdParams<Tin> p) {
   __shared__ F32ChunkOps ops[kSlots];
   __shared__ F32PrepLds prep[kSlots];
@@ -244,12 +244,12 @@ __global__ __launch_bounds__(kBlock, 1) void wkv7_fwd_f32_chunk_kernel(const F32
   const int h = blockIdx.x, b = blockIdx.y, H = p.H, T = p.T;
   const int64_t bh = (int64_t)b * H + h;
   const int64_t tstride = (int64_t)H * kHead;
-  constexpr bool kSeg = kStart == Start::kSegment;
+  constexpr bool kSeg = kStart == start::kSegment;
   const int g = kSeg ? blockIdx.z : 0, c0 = kSeg ? g * p.cps : 0;
   const int nchunks = kSeg ? min(p.cps, T / kL - c0) : T / kL;   // this segment's chunks
   const int64_t tok0 = (((int64_t)b * T + (int64_t)kL * c0) * H + h) * kHead;
   const float* const s0 = start_state<kStart>(p.s0, p.bound, bh, g);
-  const bool has_s0 = kStart == Start::kGiven || (kSeg && s0);
+  const bool has_s0 = kStart == start::kGiven || (kSeg && s0);
   const int per_ckpt = p.C / kL;
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
 
@@ -1191,8 +1191,8 @@ static hipError_t launch_fwd_f32(const ForwardDesc& d, hipStream_t stream) {
   hipError_t e = handover_fault_counter(&p.faults);
   if (e != hipSuccess) return e;
   if (d.seg.G > 1 && (e = launch_segment_bounds(d, stream)) != hipSuccess) return e;
-  auto* const kernel = d.seg.G > 1 ? wkv7_fwd_f32_chunk_kernel<Tin, Start::kSegment>
-                       : d.s0 ? wkv7_fwd_f32_chunk_kernel<Tin, Start::kGiven> : wkv7_fwd_f32_chunk_kernel<Tin, Start::kZero>;
+  auto* const kernel = d.seg.G > 1 ? wkv7_fwd_f32_chunk_kernel<Tin, start::kSegment>
+                       : d.s0 ? wkv7_fwd_f32_chunk_kernel<Tin, start::kGiven> : wkv7_fwd_f32_chunk_kernel<Tin, start::kZero>;
   hipLaunchKernelGGL(kernel, dim3(d.H, d.B, d.seg.G), dim3(kBlock), 0, stream, p);
   e = hipGetLastError();
   return e == hipSuccess && d.seg.G > 1 ? launch_segment_poison(d, stream) : e;
