@@ -99,6 +99,11 @@ def test_row_statistics_and_out_of_range_target():
     (5, 4099, "f32", 0), (520, 2057, "f32", 0), (16, 65529, "bf16", 0),
     (256, 16384, "bf16", 0), (257, 16387, "bf16", 0), (4, 16383, "f32", 0), (6, 16391, "f32", 1),
     (9, 333, "bf16", 1), (7, 2051, "f32", 3),
+    # both widths of the forward at rows of whole pieces and not, rows taken one by
+    # one (up to 512) and in pieces, each with and without blocks that share a row
+    (3, 24568, "f32", 0), (3, 24576, "bf16", 0), (2, 24576, "f32", 0), (3, 24577, "bf16", 0),
+    (5, 511, "bf16", 0), (5, 513, "f32", 0), (300, 64, "f32", 0), (2100, 48, "bf16", 0),
+    (2100, 509, "bf16", 0), (2100, 523, "bf16", 0), (300, 523, "f32", 0),
 ])
 def test_rows_that_begin_anywhere(rows, V, dt, offset):
     """Heads, pieces and tails of rows at every alignment, on both widths of the
