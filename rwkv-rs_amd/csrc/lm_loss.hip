@@ -269,7 +269,10 @@ hipError_t forward(const XentArgs& a, hipStream_t s) {
 // Blocks enough to fill the chip (eight of 256 threads a compute unit); a row has
 // at most one for each run of pieces. us without / with, bf16, 65536 logits: 16
 // rows 13.9 / 4.2, 64 rows 14.4 / 4.6, 256 rows 18.5 / 11.3, 1024 rows 46 / 44.
+// fp32 rows, twice the bytes, fill it by themselves from 512 on: 8192 logits, 256
+// rows 4.9 / 4.3, 768 rows 9.0 / 9.7, 65536 logits 22.0 / 21.6 and 83 / 86.
 constexpr int64_t kFillBlocks = 2048;
+constexpr int64_t kShareRowsF32 = 256;
 
 template <bool BF, bool kShared>
 hipError_t backward(const XentArgs& a, int form, unsigned split, hipStream_t s) {
@@ -285,7 +288,8 @@ hipError_t backward(const XentArgs& a, hipStream_t s) {
   const bool alike = ((reinterpret_cast<uintptr_t>(a.logits) ^ reinterpret_cast<uintptr_t>(a.logits_grad)) & 15) == 0;
   const int form = alike ? row_form(a.logits, a.vocab) : kElements;
   const int64_t runs = (a.vocab / (form == kElements ? 1 : kPiece) + kThreads - 1) / kThreads;
-  const int64_t split = std::max<int64_t>(1, std::min<int64_t>(kFillBlocks / a.rows, runs));
+  const int64_t fill = BF || a.rows <= kShareRowsF32 ? kFillBlocks / a.rows : 1;
+  const int64_t split = std::max<int64_t>(1, std::min<int64_t>(fill, runs));
   if (split > 1) return backward<BF, true>(a, form, static_cast<unsigned>(split), s);
   return backward<BF, false>(a, form, 1, s);
 }
