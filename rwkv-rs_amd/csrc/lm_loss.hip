@@ -228,12 +228,12 @@ __global__ __launch_bounds__(kThreads) void xent_backward_kernel(XentArgs a) {
 // A few long rows leave most of the chip idle and each is a chain of loads: four
 // times the threads a row. us, 256 / 1024 threads, bf16: 65536 logits, 64 rows
 // 11.9 / 9.1, 256 rows 12.5 / 9.6, 1024 rows 25.4 / 26.4; 32000 logits, 256 rows
-// 7.6 / 6.9 (fp32 10.0 / 7.4). At 512 rows bf16 gains 0.7-3 and fp32 loses 1.6-2;
-// at 1009 logits, where most of 1024 threads have no piece, 3.8 / 4.6. The line
-// is where every one of them has at least two.
+// 7.6 / 6.9 (fp32 10.0 / 7.4). At 512 rows bf16 gains 0.7-3 and fp32 loses 1.6-2.
+// The line is where every one of 1024 threads has at least three pieces, 24576:
+// 1 row 6.6 / 6.2, 256 rows 7.3 / 7.2; at 16384 they were 5.4 / 5.6 and 6.1 / 6.5.
 constexpr int64_t kWideRows = 256;
 constexpr int kWideThreads = 1024;
-constexpr int64_t kWideVocab = 2 * kWideThreads * kPiece;
+constexpr int64_t kWideVocab = 3 * kWideThreads * kPiece;
 
 // every row of x begins and ends on a 16-byte boundary
 bool whole_pieces(const void* x, int64_t vocab) {
