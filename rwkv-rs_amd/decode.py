@@ -203,7 +203,7 @@ def step(model, contexts, batch_ids, infer_state, context_mask,
     ids = batch_ids.to(device=dev, dtype=torch.int32).contiguous()
     elapsed = infer_state.elapsed_t.to(device=dev, dtype=torch.int32).contiguous()
     x = model.layer_norm_for_first_cell(model.embed(contexts))
-    if x.dtype != torch.float32 or x.shape != (rows, 1, C):
+    if x.dtype != torch.float32 or x.shape != (rows, 1, C) or x.device != dev:
         # the embedding and the norm have run, and run once a step
         return (model._infer_cells(x, T, batch_ids, infer_state, context_mask, unembed_mode),)
     # the cells add to it in place, and a hook or the norm itself may hold x

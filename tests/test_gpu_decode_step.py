@@ -246,6 +246,22 @@ def test_a_changed_model_still_runs(monkeypatch, request, change):
     assert all(torch.equal(x, y) for x, y in zip(st[0].state + st[0].shift_time, st[1].state + st[1].shift_time))
 
 
+def test_a_residual_stream_off_the_states_device_stays_with_the_modules(monkeypatch):
+    # here on the host: the modules refuse it; no kernel may see its address
+    announce("decode step, an embedding on the host")
+    native = load_pkg()._native
+
+    def no_library():
+        raise AssertionError("the fused step took it")
+    model = _model()
+    st = _state(model, 4, torch.float32, 1)
+    model.embed = model.embed.cpu()
+    model.layer_norm_for_first_cell = torch.nn.Identity()
+    monkeypatch.setattr(native, "lib", no_library)
+    with pytest.raises(RuntimeError, match="device"):
+        _infer(model, torch.zeros(2, 1, dtype=torch.long), torch.arange(2, device=DEV), st)
+
+
 def test_a_state_without_elapsed_t_is_refused_as_by_the_modules():
     announce("decode step, no elapsed_t")
     model = _model()
