@@ -44,8 +44,9 @@ def _plain(module, cls) -> bool:
     return not d["_forward_hooks"] and not d["_forward_pre_hooks"] and "forward" not in d
 
 
-class _Unsupported(Exception):
-    pass
+class _Unsupported(LookupError):
+    """Also what a parameter or submodule that is not there raises (KeyError is
+    a LookupError, too): both are caught where the modules are read."""
 
 
 class _Reader:
@@ -53,11 +54,11 @@ class _Reader:
     read: a plain contiguous fp32 tensor of the expected shape on the device."""
 
     def __init__(self, device):
-        self.device = device
+        self.index = device.index
 
     def tensor(self, t, shape, dtype=torch.float32) -> int:
         if (type(t) not in (nn.Parameter, torch.Tensor) or t.dtype is not dtype
-                or t.shape != shape or t.device != self.device or not t.is_contiguous()):
+                or t.shape != shape or t.get_device() != self.index or not t.is_contiguous()):
             raise _Unsupported
         p = t.data_ptr()
         if p & 15:
@@ -66,10 +67,10 @@ class _Reader:
 
     def param(self, module, name, shape) -> int:
         """A parameter; one replaced by another kind of attribute is not taken."""
-        return self.tensor(module._parameters.get(name), shape)
+        return self.tensor(module._parameters[name], shape)
 
     def linear(self, module, d_in, d_out) -> int:
-        if not _plain(module, nn.Linear) or module._parameters.get("bias", self) is not None:
+        if not _plain(module, nn.Linear) or module._parameters["bias"] is not None:
             raise _Unsupported
         return self.param(module, "weight", (d_out, d_in))
 
@@ -86,10 +87,10 @@ def _cell_params(m, cell, rd: _Reader, C: int, H: int):
     if not _plain(cell, m.CausalCell):
         raise _Unsupported
     sub = cell._modules
-    tm, cm = sub.get("time_mixer"), sub.get("channel_mixer")
+    tm, cm = sub["time_mixer"], sub["channel_mixer"]
     if not (_plain(tm, m.TimeMixer) and _plain(cm, m.ChannelMixer)):
         raise _Unsupported
-    wp, gr = tm._modules.get("weight_prepare"), tm._modules.get("gated_readout")
+    wp, gr = tm._modules["weight_prepare"], tm._modules["gated_readout"]
     if not (_plain(wp, m.WeightPrepare) and _plain(gr, m.GatedReadout)):
         raise _Unsupported
     if (not tm.neighbor_ops == wp.neighbor_ops == gr.neighbor_ops == cm.neighbor_ops == "hip"
@@ -98,40 +99,40 @@ def _cell_params(m, cell, rd: _Reader, C: int, H: int):
         raise _Unsupported
     p = _native.DecodeCellParams()
     p.norm_time_weight, p.norm_time_bias, p.norm_time_eps = rd.norm(
-        sub.get("pre_layer_norm_for_time_mix"), C)
+        sub["pre_layer_norm_for_time_mix"], C)
     p.norm_channel_weight, p.norm_channel_bias, p.norm_channel_eps = rd.norm(
-        sub.get("pre_layer_norm_for_channel_mix"), C)
+        sub["pre_layer_norm_for_channel_mix"], C)
     row = (1, 1, C)
     for i, name in enumerate(("receptance", "weight_decay", "key", "value", "learning_rate")):
         p.mix[i] = rd.param(wp, "param_" + name, row)
     p.mix[5] = rd.param(gr, "param_gate", row)
     wsub, gsub = wp._modules, gr._modules
-    p.receptance = rd.linear(wsub.get("projection_receptance"), C, C)
-    p.key = rd.linear(wsub.get("projection_key"), C, C)
-    p.value = rd.linear(wsub.get("projection_value"), C, C)
-    p.output = rd.linear(gsub.get("projection_output"), C, C)
+    p.receptance = rd.linear(wsub["projection_receptance"], C, C)
+    p.key = rd.linear(wsub["projection_key"], C, C)
+    p.value = rd.linear(wsub["projection_value"], C, C)
+    p.output = rd.linear(gsub["projection_output"], C, C)
 
     def lora(module, activation, bias):
         # the modules call the LoRA's product, or its forward, which does
         if (not _plain(module, m.LoRA) or module.activation != activation
                 or "product" in module.__dict__):
             raise _Unsupported
-        a = module._parameters.get("w_a")
+        a = module._parameters["w_a"]
         if a is None or a.dim() != 2:
             raise _Unsupported
         rank = a.shape[1]
         out = [rd.tensor(a, (C, rank)), rd.param(module, "w_b", (rank, C)), rank]
         if bias:
             out.append(rd.param(module, "bias", row))
-        elif module.__dict__.get("bias", rd) is not None:
+        elif module.__dict__["bias"] is not None:
             raise _Unsupported
         return out
     p.decay_a, p.decay_b, p.decay_rank, p.decay_bias = lora(
-        wsub.get("param_weight_decay_lora"), "tanh", True)
+        wsub["param_weight_decay_lora"], "tanh", True)
     p.rate_a, p.rate_b, p.rate_rank, p.rate_bias = lora(
-        wsub.get("param_learning_rate_lora"), "none", True)
-    p.gate_a, p.gate_b, p.gate_rank = lora(gsub.get("param_output_gate_lora"), "sigmoid", False)
-    residual = wsub.get("param_value_residual_lora") if wp.cell_id != 0 else None
+        wsub["param_learning_rate_lora"], "none", True)
+    p.gate_a, p.gate_b, p.gate_rank = lora(gsub["param_output_gate_lora"], "sigmoid", False)
+    residual = wsub["param_value_residual_lora"] if wp.cell_id != 0 else None
     if residual is not None:
         p.residual_a, p.residual_b, p.residual_rank, p.residual_bias = lora(residual, "none", True)
     elif wp.cell_id != 0:
@@ -139,15 +140,15 @@ def _cell_params(m, cell, rd: _Reader, C: int, H: int):
     p.key_removal = rd.param(wp, "param_key_removal", row)
     p.key_replacement = rd.param(wp, "param_key_replacement", row)
     p.bonus = rd.param(gr, "param_receptance_key_bonus", (H, 64))
-    gn = gsub.get("group_norm")
+    gn = gsub["group_norm"]
     if type(gn) is not nn.GroupNorm:
         raise _Unsupported
     p.group_norm_weight = rd.param(gn, "weight", (C,))
     p.group_norm_bias = rd.param(gn, "bias", (C,))
     p.group_norm_eps = m.GROUP_NORM_EPS
     p.channel_mix = rd.param(cm, "token_shift_diff_scale", row)
-    p.channel_key = rd.linear(cm._modules.get("key"), C, 4 * C)
-    p.channel_value = rd.linear(cm._modules.get("value"), 4 * C, C)
+    p.channel_key = rd.linear(cm._modules["key"], C, 4 * C)
+    p.channel_value = rd.linear(cm._modules["value"], 4 * C, C)
     for rank in (p.decay_rank, p.rate_rank, p.gate_rank, p.residual_rank or 32):
         if rank % 32 or not 0 < rank <= C:
             raise _Unsupported
@@ -196,9 +197,9 @@ def step(model, contexts, batch_ids, infer_state, context_mask,
             return None   # the first cell is the one without a value residual
         head = None
         if unembed_mode != "skip":
-            head = (rd.norm(model._modules.get("layer_norm_for_unembed"), C),
-                    rd.linear(model._modules.get("unembed"), C, model.vocab_size))
-    except _Unsupported:
+            head = (rd.norm(model._modules["layer_norm_for_unembed"], C),
+                    rd.linear(model._modules["unembed"], C, model.vocab_size))
+    except LookupError:
         return None
     ids = batch_ids.to(device=dev, dtype=torch.int32).contiguous()
     elapsed = infer_state.elapsed_t.to(device=dev, dtype=torch.int32).contiguous()
