@@ -14,8 +14,8 @@
 // registers, so no bf16 copy of them is made or kept. At 12 cells, C = 768, 8
 // sequences, vocabulary 65536, a step took 9,150 us through the modules and
 // takes 835 so. Its kernels sum to 684 us, of which the head's 201 MB of
-// weights are 49; the rest is each launch's own latency, 3-9 us (profiles/
-// rwkv7_0.1b_decode_step_kernel_stats.md). The host takes about as long.
+// weights are 49; the rest is each launch's own latency, 3-9 us. The host, which
+// reads the modules' parameters and issues them, takes about as long.
 #include "decode_launch.hpp"
 
 #include "neighbors_device.hpp"
